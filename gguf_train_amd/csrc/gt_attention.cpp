@@ -261,12 +261,14 @@ bool dispatch_forward(const AttnFwdArgs &a, int cd, int dev) {
 // Moves a device result into a new host tensor when the caller's q lives on the host.
 gt_tensor *deliver(gt_tensor *dev_t, bool to_host) { return gt_deliver(dev_t, to_host); }
 
-// Single-query attention straight from Q8_0 K/V blocks.  Returns 1 when it ran, 0 when the
-// shapes do not suit the kernel (the caller then dequantizes), -1 on error.
+// Single-query attention straight from Q8_0 K/V blocks, float16, bfloat16 or float32 queries.
+// Returns 1 when it ran, 0 when the shapes do not suit the kernel (the caller then dequantizes), -1
+// on error.
 int run_q8_decode(const gt_tensor *q, const gt_tensor *k, const gt_tensor *v, const gt_tensor *mask, float scale,
                   int is_causal, int dev, gt_tensor *o, gt_tensor *lse, Temps &tmp, const int32_t *kv_len = nullptr,
                   const int32_t *q_pos = nullptr) {
-    const gt_tensor *qs = stage(q, dev, GT_F16, tmp);
+    const int qd = q->dtype;
+    const gt_tensor *qs = stage(q, dev, qd, tmp);
     const gt_tensor *ks = k->device_type == GT_DEV_CUDA && k->device_index == dev ? k : tmp.keep(gt_to_device_dense(k, dev, -1));
     const gt_tensor *vs = v->device_type == GT_DEV_CUDA && v->device_index == dev ? v : tmp.keep(gt_to_device_dense(v, dev, -1));
     if (!qs || !ks || !vs) return -1;
@@ -276,11 +278,11 @@ int run_q8_decode(const gt_tensor *q, const gt_tensor *k, const gt_tensor *v, co
     a.lse = lse ? gt_data(lse) : nullptr;
     a.scale = scale;
     a.causal = is_causal ? 1 : 0;
-    a.out_dtype = GT_F16;
+    a.out_dtype = qd;
     a.kv_len = kv_len;
     a.q_pos = q_pos;
-    if (!attn_decode_q8_supported(a, GT_F16)) return 0;
-    if (!stage_mask(mask, dev, GT_F16, a, tmp)) return -1;
+    if (!attn_decode_q8_supported(a, qd)) return 0;
+    if (!stage_mask(mask, dev, qd, a, tmp)) return -1;
     DecodeArgs da{};
     da.f = a;
     da.nsplit = attn_decode_q8_splits(a);
@@ -410,7 +412,7 @@ int attention_forward(const char *who, const gt_tensor *q, const gt_tensor *k, c
     bool ok = true;
     int q8 = 0;  // 1: the Q8_0 decode kernel ran
     if ((o->numel > 0 || (lse && lse->numel > 0)) && k->dtype == GT_Q8_0 && v->dtype == GT_Q8_0 &&
-        q->dtype == GT_F16 && L == 1 && !o32 && !(drop && drop->on)) {
+        q->dtype != GT_F64 && L == 1 && !o32 && !(drop && drop->on)) {
         q8 = run_q8_decode(q, k, v, mask, scale, is_causal, dev, o, lse, tmp);
         ok = q8 >= 0;
     }
@@ -1478,7 +1480,7 @@ extern "C" gt_tensor *gt_kv_cache_attention(gt_kv_cache *c, const gt_tensor *q, 
     Temps tmp;
     bool ok = true;
     int q8 = 0;
-    if (o->numel > 0 && c->dtype == GT_Q8_0 && q->dtype == GT_F16 && L == 1) {
+    if (o->numel > 0 && c->dtype == GT_Q8_0 && q->dtype != GT_F64 && L == 1) {
         q8 = run_q8_decode(q, c->k, c->v, nullptr, scale, is_causal, dev, o, nullptr, tmp, kv_len, q_pos);
         ok = q8 >= 0;
     }
