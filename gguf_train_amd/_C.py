@@ -149,6 +149,10 @@ def _configure(lib: ctypes.CDLL) -> ctypes.CDLL:
     lib.gt_flash_attention_backward.argtypes = [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                                 c_void_p, c_float, c_int, p_vp, p_vp, p_vp]
     lib.gt_flash_attention_backward.restype = c_int
+    lib.gt_flash_attention_backward_as.argtypes = [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
+                                                   c_float, c_int, c_double, c_uint64, c_uint64, c_int, p_vp, p_vp,
+                                                   p_vp]
+    lib.gt_flash_attention_backward_as.restype = c_int
     lib.gt_flash_attention_noalloc.argtypes = [c_void_p, c_void_p, c_void_p, c_void_p, c_float, c_int, c_void_p]
     lib.gt_flash_attention_noalloc.restype = c_int
 

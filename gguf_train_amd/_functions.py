@@ -21,7 +21,8 @@ checkpoint's RNG-state replay reproduce the same decisions); it returns the outp
 non-differentiable log-sum-exp, from which MultiheadAttention recomputes the dropped weights.
 
 The Function subclasses torch.autograd.Function, whose engine - like the reference engine
-(gguf_train/_autograd_engine.py:325-326) - casts each gradient to its input's dtype.
+(gguf_train/_autograd_engine.py:325-326) - casts each gradient to its input's dtype; the kernels
+write that dtype themselves when q, k and v share one.
 """
 
 from __future__ import annotations
@@ -67,7 +68,7 @@ class FlashAttentionFn(torch.autograd.Function):
         if grad_out is None:
             return (None,) * 6
         q, k, v, mask, out, lse = ctx.saved_tensors
-        dq, dk, dv = _ops.flash_attention_backward(grad_out, q, k, v, mask, out, lse, ctx.scale, ctx.is_causal)
+        dq, dk, dv = _ops.input_gradients(grad_out, q, k, v, mask, out, lse, ctx.scale, ctx.is_causal)
         return (dq, dk, dv, None, None, None)
 
 
@@ -90,7 +91,7 @@ class FlashAttentionLseFn(torch.autograd.Function):
         if grad_out is None:
             return (None,) * 6
         q, k, v, mask, out, lse = ctx.saved_tensors
-        dq, dk, dv = _ops.flash_attention_backward(grad_out, q, k, v, mask, out, lse, ctx.scale, ctx.is_causal)
+        dq, dk, dv = _ops.input_gradients(grad_out, q, k, v, mask, out, lse, ctx.scale, ctx.is_causal)
         return (dq, dk, dv, None, None, None)
 
 
@@ -117,6 +118,6 @@ class FlashAttentionDropoutFn(torch.autograd.Function):
         if grad_out is None:
             return (None,) * 8
         q, k, v, mask, out, lse = ctx.saved_tensors
-        dq, dk, dv = _ops.flash_attention_dropout_backward(grad_out, q, k, v, mask, out, lse, ctx.scale,
-                                                           ctx.is_causal, *ctx.dropout)
+        dq, dk, dv = _ops.input_gradients(grad_out, q, k, v, mask, out, lse, ctx.scale, ctx.is_causal,
+                                          *ctx.dropout)
         return (dq, dk, dv, None, None, None, None, None)

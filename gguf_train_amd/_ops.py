@@ -106,6 +106,30 @@ def flash_attention_dropout_backward(dout, q, k, v, mask, out, lse, scale: float
     return adopt(pq.value, who), adopt(pk.value, who), adopt(pv.value, who)
 
 
+def input_gradients(dout, q, k, v, mask, out, lse, scale: float, is_causal: bool, p: float = 0.0, seed: int = 0,
+                    offset: int = 0):
+    """The backward as autograd hands it on: (dq, dk, dv) in the inputs' dtype when q, k and v share
+    one (the values flash_attention_backward / flash_attention_dropout_backward return, each rounded
+    once), as those return them otherwise.  p = 0: no dropout."""
+    if not (q.dtype == k.dtype == v.dtype):
+        if p == 0.0:
+            return flash_attention_backward(dout, q, k, v, mask, out, lse, scale, is_causal)
+        return flash_attention_dropout_backward(dout, q, k, v, mask, out, lse, scale, is_causal, p, seed, offset)
+    bind_stream(_device_of(q))
+    hg, hq, hk, hv = borrow(dout), borrow(q), borrow(k), borrow(v)
+    hm = borrow(mask) if mask is not None else None
+    ho = borrow(out) if out is not None else None
+    hl = borrow(lse) if lse is not None else None
+    pq, pk, pv = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_void_p()
+    rc = _C.lib.gt_flash_attention_backward_as(hg.ptr, hq.ptr, hk.ptr, hv.ptr, hm.ptr if hm else None,
+                                               ho.ptr if ho else None, hl.ptr if hl else None, ctypes.c_float(scale),
+                                               1 if is_causal else 0, float(p), _u64(seed), _u64(offset),
+                                               _GT_DTYPE[q.dtype], ctypes.byref(pq), ctypes.byref(pk), ctypes.byref(pv))
+    who = "flash_attention_backward" if p == 0.0 else "flash_attention_dropout_backward"
+    _C.check_rc(rc, who)
+    return adopt(pq.value, who), adopt(pk.value, who), adopt(pv.value, who)
+
+
 def attention_weights_dropout(q, k, mask, lse, scale: float, is_causal: bool, average_heads: bool, p: float,
                               seed: int, offset: int = 0):
     """The weights flash_attention_dropout multiplied V by (after dropout; averaged over the heads

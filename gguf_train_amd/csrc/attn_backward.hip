@@ -13,6 +13,9 @@
 //             P = exp2(S*scale*log2e - lse*log2e), dS = P * (dP - D_q)
 //             dV += P^T.dO, dK += dS^T.Q      (P, dS feed the MFMA A operand in place; dO and Q
 //                                              are read transposed from row-major LDS tiles)
+// Gradients leave as float32 or, for a caller that would round them to the inputs' dtype anyway
+// (g_half), in that dtype: the same bits without a float32 round trip through HBM (three
+// elementwise passes of 8.3 us in the training step bf16 B8 H16 L=S=1024 D64: 199 -> 180 us).
 // dK and dV of a GQA group are summed in registers (no atomics).  P and dS are split into hi +
 // lo operands so the products keep ~16 bits (bf16) or ~22 (fp16): a single fp16 operand's 2^-12
 // rounding accumulates in dV and dK, whose sums run over query rows (measured 1.27x the 2e-3
@@ -34,6 +37,7 @@
 #include "lds_dma.h"
 
 #include <cmath>
+#include <type_traits>
 
 namespace {
 
@@ -43,6 +47,14 @@ constexpr int BKV = 128;  // keys per dK/dV workgroup (32 per wavefront)
 constexpr int BQ = 64;    // query rows per dK/dV step
 constexpr int BMQ = 128;  // query rows per dQ workgroup (32 per wavefront)
 constexpr int BNK = 64;   // key rows per dQ step
+
+// x * y rounded to float32: kept in a register, or the compiler would fuse the product with a
+// conversion to float16 (v_fma_mix), whose single rounding differs from the float32 gradient's
+__device__ inline float scaled(float x, float y) {
+    float v = x * y;
+    asm("" : "+v"(v));
+    return v;
+}
 
 // ---- dK, dV ----------------------------------------------------------------------------------
 
@@ -331,19 +343,23 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void bwd_dkdv_kernel(AttnBwdA
     }
 
     // dK[key][d] (scaled) and dV[key][d]: accumulator row = key wk0 + 8(i/4) + 4half + i%4, column d
-    float *dkp = (float *)a.dk + (bk * f.S) * D;
-    float *dvp = (float *)a.dv + (bk * f.S) * D;
+    auto store = [&](auto *dkp, auto *dvp) {
+        using TG = std::remove_reference_t<decltype(*dkp)>;
 #pragma unroll
-    for (int db = 0; db < DB; ++db) {
+        for (int db = 0; db < DB; ++db) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int kr = wk0 + 8 * (i / 4) + 4 * half + (i % 4);
-            if (kr < S) {
-                dkp[(int64_t)kr * D + 32 * db + lrow] = dk[db][i] * f.scale;
-                dvp[(int64_t)kr * D + 32 * db + lrow] = dv[db][i];
+            for (int i = 0; i < 16; ++i) {
+                const int kr = wk0 + 8 * (i / 4) + 4 * half + (i % 4);
+                if (kr < S) {
+                    dkp[(int64_t)kr * D + 32 * db + lrow] = (TG)scaled(dk[db][i], f.scale);
+                    dvp[(int64_t)kr * D + 32 * db + lrow] = (TG)dv[db][i];
+                }
             }
         }
-    }
+    };
+    const int64_t base = bk * f.S * D;
+    if (a.g_half) store((T *)a.dk + base, (T *)a.dv + base);
+    else store((float *)a.dk + base, (float *)a.dv + base);
 }
 
 // ---- dQ --------------------------------------------------------------------------------------
@@ -588,14 +604,16 @@ __global__ __launch_bounds__(256, D <= 64 && (MASK == 0 || MASK == 4) ? 2 : 1) v
         __syncthreads();
     }
     if (lq < L) {
-        float *row = (float *)a.dq + (bh * f.L + lq) * D;
+        const int64_t at = (bh * f.L + lq) * D;
 #pragma unroll
         for (int db = 0; db < DB; ++db)
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
-                const f32x4 v = {dq[db][4 * g] * f.scale, dq[db][4 * g + 1] * f.scale, dq[db][4 * g + 2] * f.scale,
-                                 dq[db][4 * g + 3] * f.scale};
-                *(f32x4 *)(row + 32 * db + 8 * g + 4 * half) = v;
+                const f32x4 v = {scaled(dq[db][4 * g], f.scale), scaled(dq[db][4 * g + 1], f.scale),
+                                 scaled(dq[db][4 * g + 2], f.scale), scaled(dq[db][4 * g + 3], f.scale)};
+                const int64_t e = at + 32 * db + 8 * g + 4 * half;
+                if (a.g_half) *(u32x2 *)((T *)a.dq + e) = u32x2{M::pack(v[0], v[1]), M::pack(v[2], v[3])};
+                else *(f32x4 *)((float *)a.dq + e) = v;
             }
     }
 }

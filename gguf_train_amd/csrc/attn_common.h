@@ -90,9 +90,10 @@ struct AttnBwdArgs {
     AttnFwdArgs f;         // q/k/v/mask/o/lse as in the forward (o and lse are inputs here)
     const void *dout;      // (B,H,L,Dv) dense, compute dtype
     int o_f32;             // f.o is float32 (the training forward's unrounded output)
-    void *dq;              // (B,H,L,D) dense, float (double on the float64 path)
+    void *dq;              // (B,H,L,D) dense, float (double on the float64 path), or g_half
     void *dk;              // (B,Hkv,S,D) dense
     void *dv;              // (B,Hkv,S,Dv) dense
+    int g_half;            // fp16/bf16 MFMA kernels: dq, dk and dv are of the inputs' dtype (rounded once from float32)
     void *delta;           // (B,H,L) scratch: rowsum(P * dP)
     // dropout, MFMA kernels: (B,H,L, ceil(S/32)) words, bit j of word [row][w] = decision of key
     // 32w + j; written by the dQ kernel (which draws them), read by the dK/dV kernel

@@ -608,7 +608,7 @@ namespace {
 
 int attention_backward(const char *who, const gt_tensor *grad_out, const gt_tensor *q, const gt_tensor *k,
                        const gt_tensor *v, const gt_tensor *mask, const gt_tensor *out, const gt_tensor *lse,
-                       float scale, int is_causal, const Dropout *drop, gt_tensor **dq, gt_tensor **dk,
+                       float scale, int is_causal, const Dropout *drop, int grad_dtype, gt_tensor **dq, gt_tensor **dk,
                        gt_tensor **dv) {
     LaunchScope scope;
     if (!dq || !dk || !dv) {
@@ -638,6 +638,11 @@ int attention_backward(const char *who, const gt_tensor *grad_out, const gt_tens
     if (scale <= 0.0f) scale = 1.0f / std::sqrt((float)D);
     const int cd = compute_dtype(q, k, v);
     const int gd = cd == GT_F64 ? GT_F64 : GT_F32;
+    if (grad_dtype < 0) grad_dtype = gd;
+    if (!gt_is_float(grad_dtype)) {
+        gt_set_error(std::string(who) + ": the gradients' dtype must be a float dtype, got " + gt_dtype_name(grad_dtype));
+        return -1;
+    }
     Temps tmp;
 
     // the forward's residuals (output and log-sum-exp): given, or recomputed by a forward pass.
@@ -669,34 +674,45 @@ int attention_backward(const char *who, const gt_tensor *grad_out, const gt_tens
                 : tmp.keep(gt_to_device_dense(out, dev, od));
     if (!lse_s || !out_s) return -1;
     const int64_t qsh[4] = {B, H, L, D}, ksh[4] = {B, Hkv, S, D}, vsh[4] = {B, Hkv, S, Dv}, rsh[3] = {B, H, L};
-    gt_tensor *gq = gt_new_tensor(4, qsh, gd, GT_DEV_CUDA, dev);
-    gt_tensor *gk = gt_new_tensor(4, ksh, gd, GT_DEV_CUDA, dev);
-    gt_tensor *gv = gt_new_tensor(4, vsh, gd, GT_DEV_CUDA, dev);
+    // Gradients in the inputs' own half dtype come straight from the MFMA kernels (kd, settled
+    // before they are allocated: mfma_shape calls take those kernels unless an operand's strides or
+    // base keep them off, when the float32 gradients are converted at the end)
+    const bool half_ok = grad_dtype == cd && (cd == GT_F16 || cd == GT_BF16) && mfma_shape && L >= 1 && S >= 1 &&
+                         L < (1LL << 30) && S < (1LL << 30) && scale > 0.0f;
     gt_tensor *delta = tmp.keep(gt_new_tensor(3, rsh, gd, GT_DEV_CUDA, dev));
     const gt_tensor *qs = stage(q, dev, cd, tmp), *ks = stage(k, dev, cd, tmp), *vs = stage(v, dev, cd, tmp);
     const gt_tensor *gos = grad_out->device_type == GT_DEV_CUDA && grad_out->device_index == dev &&
                                    grad_out->dtype == cd && gt_is_dense(grad_out)
                                ? grad_out
                                : tmp.keep(gt_to_device_dense(grad_out, dev, cd));
-    bool ok = gq && gk && gv && delta && qs && ks && vs && gos && lse_s;
+    bool ok = delta && qs && ks && vs && gos && lse_s;
     AttnBwdArgs a{};
     if (ok) {
         fill_qkv(a.f, qs, ks, vs);
         ok = stage_mask(mask, dev, cd, a.f, tmp);
     }
+    gt_tensor *gq = nullptr, *gk = nullptr, *gv = nullptr;
     if (ok) {
         a.f.lse = gt_data(lse_s);
         a.f.scale = scale;
         a.f.causal = is_causal ? 1 : 0;
         a.f.out_dtype = cd;
         a.dout = gt_data(gos);
-        a.dq = gt_data(gq);
-        a.dk = gt_data(gk);
-        a.dv = gt_data(gv);
         a.delta = gt_data(delta);
         a.f.o = const_cast<void *>(gt_data(out_s));
         a.o_f32 = od == GT_F32 && cd != GT_F32;
         apply_dropout(a.f, drop);
+        a.g_half = half_ok && (Dp || attn_bwd_mfma_supported(a, cd)) ? 1 : 0;
+        const int kd = a.g_half ? cd : gd;
+        gq = gt_new_tensor(4, qsh, kd, GT_DEV_CUDA, dev);
+        gk = gt_new_tensor(4, ksh, kd, GT_DEV_CUDA, dev);
+        gv = gt_new_tensor(4, vsh, kd, GT_DEV_CUDA, dev);
+        ok = gq && gk && gv;
+    }
+    if (ok) {
+        a.dq = gt_data(gq);
+        a.dk = gt_data(gk);
+        a.dv = gt_data(gv);
         // heads padded to the MFMA kernels' sizes: padded inputs, padded gradients unpadded after.
         // Float32: only where its MFMA backward takes the padded call
         if (cd == GT_F32 && !f32_pads(a.f)) Dp = 0;
@@ -706,9 +722,9 @@ int attention_backward(const char *who, const gt_tensor *grad_out, const gt_tens
             const gt_tensor *vp = pad_heads(vs, Dp, dev, tmp), *gp = pad_heads(gos, Dp, dev, tmp);
             const gt_tensor *op = pad_heads(out_s, Dp, dev, tmp);
             const int64_t qsh2[4] = {B, H, L, Dp}, ksh2[4] = {B, Hkv, S, Dp};
-            pq = tmp.keep(gt_new_tensor(4, qsh2, gd, GT_DEV_CUDA, dev));
-            pk = tmp.keep(gt_new_tensor(4, ksh2, gd, GT_DEV_CUDA, dev));
-            pv = tmp.keep(gt_new_tensor(4, ksh2, gd, GT_DEV_CUDA, dev));
+            pq = tmp.keep(gt_new_tensor(4, qsh2, gq->dtype, GT_DEV_CUDA, dev));
+            pk = tmp.keep(gt_new_tensor(4, ksh2, gq->dtype, GT_DEV_CUDA, dev));
+            pv = tmp.keep(gt_new_tensor(4, ksh2, gq->dtype, GT_DEV_CUDA, dev));
             ok = qp && kp && vp && gp && op && pq && pk && pv;
             if (ok) {
                 fill_qkv(a.f, qp, kp, vp);
@@ -733,12 +749,22 @@ int attention_backward(const char *who, const gt_tensor *grad_out, const gt_tens
                 note_launch(std::string("backward mfma ") + dtype_tag(cd) + " D=" + std::to_string(a.f.D) +
                             (cd == GT_F32 && attn_bwd_f32_split(a) ? " split" : ""));
             ok = ok && gt_hip_check(launch_attn_bwd_mfma(a, cd, gt_stream()), "flash_attention_backward kernel");
+        } else if (ok && a.g_half) {  // half_ok covers what the padded call is checked for
+            gt_set_error(std::string(who) + ": the padded call does not suit the MFMA kernels");
+            ok = false;
         } else if (ok) {
             note_launch(std::string("backward generic ") + dtype_tag(cd));
             ok = gt_hip_check(launch_attn_generic_bwd(a, cd, gt_stream()), "flash_attention_backward kernel");
         }
         if (ok && Dp) ok = unpad_heads(pq, gq) && unpad_heads(pk, gk) && unpad_heads(pv, gv);
     }
+    for (gt_tensor **g : {&gq, &gk, &gv})
+        if (ok && (*g)->dtype != grad_dtype) {
+            gt_tensor *c = gt_to_device_dense(*g, dev, grad_dtype);
+            gt_tensor_free(*g);
+            *g = c;
+            ok = c != nullptr;
+        }
     if (ok) {
         gq = deliver(gq, host_io);
         gk = deliver(gk, host_io);
@@ -763,8 +789,27 @@ extern "C" int gt_flash_attention_backward(const gt_tensor *grad_out, const gt_t
                                            const gt_tensor *v, const gt_tensor *mask, const gt_tensor *out,
                                            const gt_tensor *lse, float scale, int is_causal, gt_tensor **dq,
                                            gt_tensor **dk, gt_tensor **dv) {
-    return attention_backward("flash_attention_backward", grad_out, q, k, v, mask, out, lse, scale, is_causal, nullptr,
+    return attention_backward("flash_attention_backward", grad_out, q, k, v, mask, out, lse, scale, is_causal, nullptr, -1,
                               dq, dk, dv);
+}
+
+extern "C" int gt_flash_attention_backward_as(const gt_tensor *grad_out, const gt_tensor *q, const gt_tensor *k,
+                                              const gt_tensor *v, const gt_tensor *mask, const gt_tensor *out,
+                                              const gt_tensor *lse, float scale, int is_causal, double dropout_p,
+                                              uint64_t seed, uint64_t offset, int grad_dtype, gt_tensor **dq,
+                                              gt_tensor **dk, gt_tensor **dv) {
+    const char *who = dropout_p == 0.0 ? "flash_attention_backward" : "flash_attention_dropout_backward";
+    if (dq) *dq = nullptr;
+    if (dk) *dk = nullptr;
+    if (dv) *dv = nullptr;
+    if (grad_dtype < 0) {
+        gt_set_error(std::string(who) + ": the gradients' dtype must be a float dtype");
+        return -1;
+    }
+    Dropout drop;
+    if (!make_dropout(who, dropout_p, seed, offset, drop)) return -1;
+    return attention_backward(who, grad_out, q, k, v, mask, out, lse, scale, is_causal, drop.on ? &drop : nullptr,
+                              grad_dtype, dq, dk, dv);
 }
 
 // ---- dropout ------------------------------------------------------------------------------------
@@ -801,7 +846,7 @@ extern "C" int gt_flash_attention_dropout_backward(const gt_tensor *grad_out, co
     if (dv) *dv = nullptr;
     Dropout drop;
     if (!make_dropout(who, dropout_p, seed, offset, drop)) return -1;
-    return attention_backward(who, grad_out, q, k, v, mask, out, lse, scale, is_causal, &drop, dq, dk, dv);
+    return attention_backward(who, grad_out, q, k, v, mask, out, lse, scale, is_causal, &drop, -1, dq, dk, dv);
 }
 
 // The dropout decisions themselves, (B,H,L,S) bool on device `device_index` (1 = kept): the

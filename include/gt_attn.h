@@ -231,6 +231,17 @@ GT_API int gt_flash_attention_dropout(const gt_tensor *q, const gt_tensor *k, co
                                       uint64_t seed, uint64_t offset, gt_tensor **out, gt_tensor **lse,
                                       gt_tensor **out32);
 
+/* No counterpart in the reference, whose engine casts each gradient to its input's dtype after the
+ * backward (gguf_train/_autograd_engine.py:325-326): gt_flash_attention_backward (dropout_p = 0; seed
+ * and offset unused then) or gt_flash_attention_dropout_backward with the gradients in `grad_dtype`,
+ * each value rounded once from the one those return.  For float16/bfloat16 inputs and their own
+ * dtype the kernels write it themselves.  Returns 0 on success. */
+GT_API int gt_flash_attention_backward_as(const gt_tensor *grad_out, const gt_tensor *q, const gt_tensor *k,
+                                          const gt_tensor *v, const gt_tensor *mask, const gt_tensor *out,
+                                          const gt_tensor *lse, float scale, int is_causal, double dropout_p,
+                                          uint64_t seed, uint64_t offset, int grad_dtype, gt_tensor **dq,
+                                          gt_tensor **dk, gt_tensor **dv);
+
 /* The backward of gt_flash_attention_dropout with the same (dropout_p, seed, offset): the
  * gradients of the reference's composition under the same dropout decisions, as
  * gt_flash_attention_backward otherwise (out / lse may be NULL: recomputed). */
