@@ -5,9 +5,9 @@
 // attend to -> 0, output rounded from fp32 to the input dtype.
 //
 // Workgroup: 4 wavefronts, query tiles of BM = 128 rows (32 per wavefront), two workgroups per
-// CU (two wavefronts per SIMD), so each K/V tile brought into LDS serves 128 queries.  A workgroup runs the query tiles p and
-// nq-1-p of one head one after the other: under the causal mask their key ranges add up to
-// the same length for every p, so all workgroups carry equal work.  K/V tiles of BN = 64 rows
+// CU (two wavefronts per SIMD), so each K/V tile brought into LDS serves 128 queries.  A workgroup
+// runs one query tile, or the tiles p and nq-1-p of one head one after the other: under the causal
+// mask their key ranges add up to the same length for every p (tile_order).  K/V tiles of BN = 64 rows
 // stream through NST LDS stages: global_load_lds_dwordx4 writes tile s+NST-1 straight into LDS
 // (no staging registers) while tile s is computed, with one barrier per tile; the loads are
 // issued after tile s's S MFMAs (2-3% faster on the prefill workload than right after the
@@ -125,6 +125,56 @@ __device__ inline void rope_rows(typename Mfma<T>::V8 *q, const float2 *tab, int
     }
 }
 
+// How a launch deals query tiles to workgroups.  kPairs: tiles p and nq-1-p of a head, one after
+// the other (equal work for every workgroup under the causal mask).  kSingle: one tile each, the
+// heaviest first (kHeadMajor: no causal mask, a head's tiles together); kFolded: one tile each where
+// all workgroups are resident at once, the heavier half first and then the lighter half from its
+// lightest, so that the two workgroups of a CU carry about the same together.
+enum TileOrder { kPairs = 0, kSingle = 1, kFolded = 2, kHeadMajor = 3 };
+
+// The tile(s) and head of workgroup x: qa (and then qb, when it differs).
+struct TileOf {
+    int qa, qb;
+    int64_t bh;
+};
+__device__ inline TileOf tile_of(int order, int nq, int64_t BH, uint32_t x) {
+    // Workgroups are dealt to the 8 XCDs round robin (x % 8); when the heads split evenly,
+    // XCD x takes heads [x*BH/8, (x+1)*BH/8), so their K/V stay in its own L2.
+    const bool even = BH % 8 == 0;
+    const int64_t heads = even ? BH / 8 : BH, i = even ? x / 8 : x, h0 = even ? (int64_t)(x % 8) * heads : 0;
+    if (order == kPairs) {
+        const int npairs = (nq + 1) / 2, p = (int)(i % npairs);
+        return {nq - 1 - p, p, h0 + i / npairs};
+    }
+    if (order == kHeadMajor) {
+        const int t = (int)(i % nq);
+        return {t, t, h0 + i / nq};
+    }
+    const int r = (int)(i / heads);  // rank of the tile
+    int t = nq - 1 - r;
+    if (order == kFolded && r >= (nq + 1) / 2) t = r - (nq + 1) / 2;
+    return {t, t, h0 + i % heads};
+}
+
+// Resident workgroups of the prefill kernels: two on each of the 256 CUs.
+constexpr int64_t kPrefillSlots = 512;
+
+// Pairs keep every workgroup's work equal and load Q and set up half as often, so they are taken
+// where their rounds over the slots are nearly full (causal fp16 B4 H32 L=S=2048 D128, two full
+// rounds: 162 us, single tiles 171).  Fewer workgroups than that leave slots empty, and a second
+// workgroup's MFMAs no longer cover the first one's softmax: single tiles then (same box, pairs
+// against single: bf16 B1 H32/8 L=S=2048 D128 68.2 -> 64.9 us, fp16 B1 H32/8 L=S=1024 32.2 -> 26.8,
+// fp16 B1 H8 L=S=3000 67.4 -> 58.8).  Without the causal mask all tiles weigh the same and single
+// ones always spread better (fp16 B4 H32/8 L500 S1500 D128 72.3 -> 60.3 us, with an (L,S) mask 132.8
+// -> 93.0; bf16 B2 H16 L300 S900 D64 34.5 -> 20.0; B4 H32 L=S=2048, many rounds: even).
+inline TileOrder tile_order(const AttnFwdArgs &a, int nq) {
+    const int64_t BH = a.B * a.H, pairs = (int64_t)((nq + 1) / 2) * BH;
+    if (!a.causal) return kHeadMajor;
+    const int64_t rounds = (pairs + kPrefillSlots - 1) / kPrefillSlots;
+    if (nq == 1 || pairs * 16 >= rounds * kPrefillSlots * 15) return kPairs;
+    return nq * BH <= kPrefillSlots ? kFolded : kSingle;
+}
+
 // Keys covered by query tile qt: the sequence's keys, or (causal) up to the tile's last row,
 // whose position is qpos + qt*BM + BM-1.
 template <bool CAUSAL, int BM, int BN>
@@ -145,7 +195,7 @@ __device__ inline int key_tiles(int qt, int nkv, int qpos) {
 // exact to ~22 bits instead of fp16's 11.
 template <typename T, int D, bool CAUSAL, int MASK, bool ROPE = false, bool DROP = false, bool HILO = false>
 __global__ __launch_bounds__(64 * nw_of<D>(), DROP && (MASK == 1 || MASK == 2 || MASK >= 5) ? 1 : 8 / nw_of<D>()) void prefill_fwd_kernel(
-    AttnFwdArgs a, int nq, int npairs) {
+    AttnFwdArgs a, int nq, int order) {
     constexpr int NW = nw_of<D>(), BM = bm_of<D>(), NST = nst_of<D>(), BN = bn_of<D>();
     constexpr int NKB = BN / 32;  // 32-key blocks per tile
     using M = Mfma<T>;
@@ -169,25 +219,14 @@ __global__ __launch_bounds__(64 * nw_of<D>(), DROP && (MASK == 1 || MASK == 2 ||
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wavefront index, uniform
     const int lrow = lane & 31, half = lane >> 5;
     const int g16 = lane >> 4, i16 = lane & 15;
-    const int64_t BH = a.B * a.H;
-    // Workgroups are dealt to the 8 XCDs round robin (x % 8); when the heads split evenly,
-    // XCD x takes heads [x*BH/8, (x+1)*BH/8), so their K/V stay in its own L2.
-    int pair;
-    int64_t bh;
-    if (BH % 8 == 0) {
-        const int64_t hpx = BH / 8, i = blockIdx.x / 8;
-        pair = (int)(i % npairs);
-        bh = (int64_t)(blockIdx.x % 8) * hpx + i / npairs;
-    } else {
-        pair = (int)(blockIdx.x % npairs);
-        bh = (int64_t)blockIdx.x / npairs;
-    }
+    const TileOf tile = tile_of(order, nq, a.B * a.H, blockIdx.x);
+    const int64_t bh = tile.bh;
     const int64_t b = bh / a.H, h = bh % a.H, hk = h / (a.H / a.Hkv);
     const int L = (int)a.L, S = (int)a.S;
     // keys present for this sequence and the position of its query row 0 (KV cache; the
     // reference operator: S and 0)
     const int nkv = attn_kv_len(a, b), qpos = attn_q_pos(a, b);
-    const int qa = nq - 1 - pair, qb = pair;  // the heavier tile first
+    const int qa = tile.qa, qb = tile.qb;  // the heavier tile first
     const int nparts = qa == qb ? 1 : 2;
     const int na = key_tiles<CAUSAL, BM, BN>(qa, nkv, qpos);
     const int total = na + (nparts == 2 ? key_tiles<CAUSAL, BM, BN>(qb, nkv, qpos) : 0);
@@ -516,16 +555,16 @@ __global__ __launch_bounds__(64 * nw_of<D>(), DROP && (MASK == 1 || MASK == 2 ||
 }
 
 template <typename T, int D>
-hipError_t launch_variant(const AttnFwdArgs &a, int nq, int npairs, int64_t grid, hipStream_t s) {
+hipError_t launch_variant(const AttnFwdArgs &a, int nq, int order, int64_t grid, hipStream_t s) {
     const int mode = attn_mask_mode(a);
 #define GT_PREFILL_LAUNCH(C, MK) \
-    hipLaunchKernelGGL((prefill_fwd_kernel<T, D, C, MK>), dim3((unsigned)grid), dim3(64 * nw_of<D>()), 0, s, a, nq, npairs)
+    hipLaunchKernelGGL((prefill_fwd_kernel<T, D, C, MK>), dim3((unsigned)grid), dim3(64 * nw_of<D>()), 0, s, a, nq, order)
 #define GT_PREFILL_LAUNCH_R(C, MK) \
-    hipLaunchKernelGGL((prefill_fwd_kernel<T, D, C, MK, true>), dim3((unsigned)grid), dim3(64 * nw_of<D>()), 0, s, a, nq, npairs)
+    hipLaunchKernelGGL((prefill_fwd_kernel<T, D, C, MK, true>), dim3((unsigned)grid), dim3(64 * nw_of<D>()), 0, s, a, nq, order)
 #define GT_PREFILL_LAUNCH_D(C, MK) \
-    hipLaunchKernelGGL((prefill_fwd_kernel<T, D, C, MK, false, true, std::is_same<T, _Float16>::value>), dim3((unsigned)grid), dim3(64 * nw_of<D>()), 0, s, a, nq, npairs)
+    hipLaunchKernelGGL((prefill_fwd_kernel<T, D, C, MK, false, true, std::is_same<T, _Float16>::value>), dim3((unsigned)grid), dim3(64 * nw_of<D>()), 0, s, a, nq, order)
 #define GT_PREFILL_LAUNCH_X(C, MK) \
-    hipLaunchKernelGGL((prefill_fwd_kernel<T, D, C, MK, false, false, true>), dim3((unsigned)grid), dim3(64 * nw_of<D>()), 0, s, a, nq, npairs)
+    hipLaunchKernelGGL((prefill_fwd_kernel<T, D, C, MK, false, false, true>), dim3((unsigned)grid), dim3(64 * nw_of<D>()), 0, s, a, nq, order)
     if (a.dropout) {
         if (a.rope_q) return hipErrorInvalidValue;  // dropout runs on unrotated queries only
         if (a.causal) {
@@ -1166,13 +1205,13 @@ hipError_t launch_attn_prefill(const AttnFwdArgs &a, int cd, hipStream_t s) {
     if (attn_prefill_asm_supported(a, cd)) return launch_attn_prefill_asm(a, s);
     const int BM = a.D == 64 ? bm_of<64>() : bm_of<128>();
     const int nq = (int)((a.L + BM - 1) / BM);
-    const int npairs = (nq + 1) / 2;  // query tiles p and nq-1-p share a workgroup
-    const int64_t grid = (int64_t)npairs * a.B * a.H;
+    const int order = tile_order(a, nq);
+    const int64_t grid = (int64_t)(order == kPairs ? (nq + 1) / 2 : nq) * a.B * a.H;
     if (grid <= 0) return hipSuccess;
     if (grid > 0x7fffffffLL) return hipErrorInvalidConfiguration;
     if (cd == GT_F16)
-        return a.D == 128 ? launch_variant<_Float16, 128>(a, nq, npairs, grid, s)
-                          : launch_variant<_Float16, 64>(a, nq, npairs, grid, s);
-    return a.D == 128 ? launch_variant<__bf16, 128>(a, nq, npairs, grid, s)
-                      : launch_variant<__bf16, 64>(a, nq, npairs, grid, s);
+        return a.D == 128 ? launch_variant<_Float16, 128>(a, nq, order, grid, s)
+                          : launch_variant<_Float16, 64>(a, nq, order, grid, s);
+    return a.D == 128 ? launch_variant<__bf16, 128>(a, nq, order, grid, s)
+                      : launch_variant<__bf16, 64>(a, nq, order, grid, s);
 }

@@ -1,0 +1,48 @@
+"""Every way the half-precision prefill deals query tiles to workgroups (pairs of tiles, single tiles
+heaviest first, single tiles folded, head by head), with heads that do and do not divide among the 8
+XCDs and odd tile counts, against the float64 oracle on a few heads; every row of every head is also
+checked to be written (the output buffer holds other calls' values before)."""
+
+import pytest
+import torch
+
+import gguf_train_amd as g
+
+from _util import assert_close, oracle_forward, randn
+
+pytestmark = pytest.mark.gpu
+
+
+def _order(causal, nq, heads):
+    """The rule under test, restated: 512 resident workgroups."""
+    pairs = (nq + 1) // 2 * heads
+    if not causal:
+        return "head major"
+    if nq == 1 or pairs * 16 >= (pairs + 511) // 512 * 512 * 15:
+        return "pairs"
+    return "folded" if nq * heads <= 512 else "single"
+
+
+@pytest.mark.parametrize("dtype,B,H,Hkv,L,S,D,causal,order", [
+    (torch.float16, 1, 3, 1, 300, 300, 128, True, "folded"),
+    (torch.bfloat16, 2, 8, 4, 257, 400, 64, True, "folded"),
+    (torch.float16, 1, 8, 2, 129, 129, 64, True, "folded"),
+    (torch.float16, 1, 32, 32, 2300, 300, 64, True, "single"),
+    (torch.bfloat16, 1, 36, 12, 2305, 200, 64, True, "single"),
+    (torch.float16, 4, 64, 64, 500, 200, 64, True, "pairs"),
+    (torch.float16, 2, 5, 5, 128, 128, 128, True, "pairs"),
+    (torch.bfloat16, 1, 6, 2, 400, 130, 128, False, "head major"),
+    (torch.float16, 2, 8, 8, 385, 100, 64, False, "head major"),
+])
+def test_every_tile_order(dev, dtype, B, H, Hkv, L, S, D, causal, order):
+    assert _order(causal, (L + 127) // 128, B * H) == order
+    q, k, v = (randn((B, h, n, D), i + L, dtype) for i, (h, n) in enumerate(((H, L), (Hkv, S), (Hkv, S))))
+    poison = torch.full((B, H, L, D), float("nan"), dtype=dtype, device=dev)
+    del poison  # its block is what the output gets next: rows nobody wrote would be NaN
+    got = g.flash_attention(q.to(dev), k.to(dev), v.to(dev), None, 0.0, causal)
+    assert torch.isfinite(got).all()
+    G = H // Hkv
+    for b, h in {(0, 0), (B - 1, H - 1), (0, H // 2)}:
+        kv = slice(h // G, h // G + 1)
+        want = oracle_forward(q[b:b + 1, h:h + 1], k[b:b + 1, kv], v[b:b + 1, kv], is_causal=causal)
+        assert_close(got[b:b + 1, h:h + 1], want, dtype, f"head {b},{h}")
