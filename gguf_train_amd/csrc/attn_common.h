@@ -19,6 +19,19 @@
 
 #include "gt_philox.h"
 
+// Classes of a mask's tiles (attn_mask_tiles.hip): 128 query rows x the prefill kernel's key tile.
+constexpr int kMaskTileRows = 128;
+constexpr int kMaskTilesMax = 1024;  // key tiles per row that the prefill kernel's list holds
+enum AttnMaskClass { kMaskTileClear = 0, kMaskTileBlocked = 1, kMaskTileBits = 2, kMaskTileValues = 3 };
+struct AttnMaskTiles {
+    const uint8_t *cls;    // (batches, query tiles, nkt); null: no classes
+    const uint32_t *bits;  // (batches, L, words): bit j of word w = key 32w + j is not blocked
+    int nkt, words;
+    int batched;           // 1: a mask per sequence, 0: one for all
+};
+// Row pitch (floats) of the float32 copy of a half-precision mask: whole 4-key groups.
+__host__ __device__ inline int64_t attn_mask_copy_pitch(int64_t S) { return (S + 3) / 4 * 4; }
+
 struct AttnFwdArgs {
     const void *q;
     const void *k;
@@ -49,13 +62,17 @@ struct AttnFwdArgs {
     // log-sum-exp stays that of the undropped scores.  Decode kernels never see it.
     int dropout;
     GtDropout drop;
+    // Tile classes of the mask (mask mode 7, prefill only; mask, m_sb and m_sl then describe its float32
+    // values, read where a tile has others than 0 and -inf).
+    AttnMaskTiles mt;
 };
 
 // Mask mode of the MFMA kernels: 0 none; 1 bool bytes, 2 additive float (per element, any
 // strides); 4 additive float that does not depend on the query row (key padding); 5 / 6 bool /
 // float per element with contiguous keys, rows and broadcast strides of whole 4-key groups and
-// an aligned base (4-key loads).
+// an aligned base (4-key loads); 7 tile classes (a.mt).
 inline int attn_mask_mode(const AttnFwdArgs &a) {
+    if (a.mt.cls) return 7;
     if (!a.mask) return 0;
     if (!a.mask_bool && a.m_sl == 0) return 4;
     const bool vec = a.m_ss == 1 && a.S >= 4 && a.S % 4 == 0 && a.m_sb % 4 == 0 && a.m_sh % 4 == 0 &&
@@ -163,6 +180,11 @@ bool attn_prefill_supported(const AttnFwdArgs &f, int cd);
 // (launch_attn_prefill runs the software-pipelined fp16 head-size-128 kernel where
 // attn_prefill_asm_supported holds, the HIP prefill kernel otherwise)
 hipError_t launch_attn_prefill(const AttnFwdArgs &a, int cd, hipStream_t s);
+int attn_prefill_key_tile(const AttnFwdArgs &f);  // keys per tile of the half-precision kernel
+// Fills t.cls and t.bits from a mask of `batches` (L, S) planes; kind 0 bool bytes, 1 float16, 2
+// bfloat16, 3 float32; copy: float32 values of the half-precision kinds' kMaskTileValues tiles.
+hipError_t launch_attn_mask_tiles(int kind, const void *mask, int64_t batches, int64_t sb, int64_t sl, int64_t ss,
+                                  int64_t L, int64_t S, int bn, const AttnMaskTiles &t, float *copy, hipStream_t s);
 bool attn_prefill_asm_supported(const AttnFwdArgs &f, int cd);
 bool attn_prefill_f32_split(const AttnFwdArgs &f, int cd);  // float32: the small-grid kernel
 hipError_t launch_attn_prefill_asm(const AttnFwdArgs &a, hipStream_t s);

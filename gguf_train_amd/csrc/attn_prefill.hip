@@ -186,7 +186,10 @@ __device__ inline int key_tiles(int qt, int nkv, int qpos) {
 // MASK: 0 = none, 1 = bool bytes, 2 = additive float, 4 = additive float that does not depend
 // on the query row (key padding: the tile's mask row travels to LDS with the K/V tile),
 // 5 / 6 = bool / float with contiguous keys and 4-key aligned rows: a lane's 4 consecutive keys
-// in one 4- / 16-byte load, issued with the tile's DMA so that they land during S = K.Q^T.
+// in one 4- / 16-byte load, issued with the tile's DMA so that they land during S = K.Q^T;
+// 7 = tile classes (attn_mask_tiles.hip): the workgroup lists the key tiles that are not blocked
+// throughout and walks that list; a tile that blocks nothing takes no mask work, one that only
+// blocks one bit per score, loaded a tile ahead, other tiles the float loads of mode 6.
 // (dropout with a per-element mask: one workgroup per CU is the guaranteed minimum, so that the
 // Philox state does not spill)
 // HILO (fp16 training forwards, with and without dropout): P enters P.V as hi + lo fp16 operands
@@ -206,14 +209,17 @@ __global__ __launch_bounds__(64 * nw_of<D>(), DROP && (MASK == 1 || MASK == 2 ||
     constexpr int TILE = BN * D;           // elements per tile
     constexpr int NPW = BN * CH / 64 / NW; // 1 KB wave loads per operand, wave and tile
     constexpr bool MROW = MASK == 4;
-    constexpr bool MVEC = MASK >= 5;                     // per-element mask, 4 keys per load
+    constexpr bool MVEC = MASK == 5 || MASK == 6;        // per-element mask, 4 keys per load
     constexpr bool MBOOL = MASK == 1 || MASK == 5;
+    constexpr bool MTILE = MASK == 7;
     constexpr int PER = 2 * NPW + (MROW ? BN / 64 : 0);  // loads per wave and tile (K, V, mask row)
     static_assert(NPW >= 1 && PER * (NST - 2) < 64, "tile split");
     static_assert(BN % 64 == 0, "mask row: one key per lane and load");
     __shared__ __attribute__((aligned(1024))) T sK[NST][TILE];
     __shared__ __attribute__((aligned(1024))) T sV[NST][TILE];
     __shared__ __attribute__((aligned(16))) float sMk[MROW ? NST : 1][BN];
+    __shared__ uint16_t sList[MTILE ? 2 * kMaskTilesMax : 1];  // key tile | class << 14, both parts'
+    static_assert(!MTILE || BM == kMaskTileRows, "mask tile rows");
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wavefront index, uniform
@@ -228,8 +234,30 @@ __global__ __launch_bounds__(64 * nw_of<D>(), DROP && (MASK == 1 || MASK == 2 ||
     const int nkv = attn_kv_len(a, b), qpos = attn_q_pos(a, b);
     const int qa = tile.qa, qb = tile.qb;  // the heavier tile first
     const int nparts = qa == qb ? 1 : 2;
-    const int na = key_tiles<CAUSAL, BM, BN>(qa, nkv, qpos);
-    const int total = na + (nparts == 2 ? key_tiles<CAUSAL, BM, BN>(qb, nkv, qpos) : 0);
+    int na = key_tiles<CAUSAL, BM, BN>(qa, nkv, qpos);
+    int total = na + (nparts == 2 ? key_tiles<CAUSAL, BM, BN>(qb, nkv, qpos) : 0);
+    const int64_t mtb = MTILE && a.mt.batched ? b : 0;  // the mask's batch index
+    if constexpr (MTILE) {
+        // every wave forms the same counts, wave 0 writes the list
+        int n = 0;
+        for (int part = 0; part < nparts; ++part) {
+            const int qt = part == 0 ? qa : qb, cand = part == 0 ? na : total - na;
+            const uint8_t *cls = a.mt.cls + (mtb * nq + qt) * a.mt.nkt;
+            const int first = n;
+            for (int t0 = 0; t0 < cand; t0 += 64) {
+                const int c = t0 + lane < cand ? cls[t0 + lane] : kMaskTileBlocked;
+                const uint64_t keep = __builtin_amdgcn_ballot_w64(c != kMaskTileBlocked);
+                if (w == 0 && c != kMaskTileBlocked)
+                    sList[n + __builtin_popcountll(keep & ((1ull << lane) - 1))] = (uint16_t)((t0 + lane) | c << 14);
+                n += __builtin_popcountll(keep);
+            }
+            if (part == 0) total -= na - (n - first), na = n - first;
+            else total = n;
+        }
+        __syncthreads();
+    }
+    // the list's entry of a flat step (uniform)
+    auto entry = [&](int step) { return (int)__builtin_amdgcn_readfirstlane((int)sList[step]); };
 
     const T *kbase = (const T *)a.k + b * a.k_sb + hk * a.k_sh;
     const T *vbase = (const T *)a.v + b * a.v_sb + hk * a.v_sh;
@@ -259,9 +287,21 @@ __global__ __launch_bounds__(64 * nw_of<D>(), DROP && (MASK == 1 || MASK == 2 ||
         vofs_n[n] = (uint32_t)lrow_n[n] * v_row + lcol_n[n];
     }
     const float *mrow = MROW ? (const float *)a.mask + b * a.m_sb + h * a.m_sh : nullptr;
+    // MTILE: bits of the keys of the step to come, one word per 32 keys of this lane's row
+    uint32_t nbits[MTILE ? NKB : 1];
     auto issue = [&](int step) {
-        const int kt = step < na ? step : step - na;
+        int kt = step < na ? step : step - na;
         const int st = step % NST;
+        if constexpr (MTILE) {
+            const int e = entry(step);
+            kt = e & 0x3fff;
+            if (e >> 14 == kMaskTileBits) {
+                const int row = min((step < na ? qa : qb) * BM + 32 * w + lrow, L - 1);
+                const uint32_t *wd = a.mt.bits + (mtb * L + row) * a.mt.words;
+#pragma unroll
+                for (int kb = 0; kb < NKB; ++kb) nbits[kb] = wd[min(kt * NKB + kb, a.mt.words - 1)];
+            }
+        }
         if constexpr (MROW) {
             // the mask values of keys kt*BN .. +63 (keys past S repeat key S-1); every wave writes
             // the same row, which keeps the loads per wave and tile uniform and needs no exec mask
@@ -352,7 +392,8 @@ __global__ __launch_bounds__(64 * nw_of<D>(), DROP && (MASK == 1 || MASK == 2 ||
         const int64_t mrb = MVEC ? b * a.m_sb + h * a.m_sh + (int64_t)min(lq, L - 1) * a.m_sl : 0;
 
         for (int j = 0; j < ntiles; ++j, ++step) {
-            const int k0 = j * BN;
+            const int ent = MTILE ? entry(step) : j;
+            const int k0 = (MTILE ? ent & 0x3fff : j) * BN, mcls = MTILE ? ent >> 14 : 0;
             // Tile `step` is complete once at most the loads of the tiles issued after it are
             // outstanding (vector memory loads complete in order); the barrier then makes every
             // wavefront's part visible and guarantees stage (step-1) % NST is no longer read.
@@ -366,6 +407,11 @@ __global__ __launch_bounds__(64 * nw_of<D>(), DROP && (MASK == 1 || MASK == 2 ||
             if constexpr (D <= 64) progress_priority(step);
             const T *cK = sK[step % NST];
             const T *cV = sV[step % NST];
+            uint32_t mbits[MTILE ? NKB : 1];  // this tile's bits, at this lane's first key
+            if constexpr (MTILE) {
+#pragma unroll
+                for (int kb = 0; kb < NKB; ++kb) mbits[kb] = nbits[kb] >> (4 * half);
+            }
             // MVEC: keys k0 + 32kb + 8g + 4half + 0..3 of this lane's row (starts past the last
             // 4 keys read those: their scores are blocked below)
             f32x4 mvf[MVEC && !MBOOL ? NKB : 1][4];
@@ -412,7 +458,29 @@ __global__ __launch_bounds__(64 * nw_of<D>(), DROP && (MASK == 1 || MASK == 2 ||
 
             // ---- masks: s[kb][i] is (key = k0 + 32kb + 8(i/4) + 4half + i%4, query = lq) ----
             const bool edge = k0 + BN > nkv || (CAUSAL && k0 + BN - 1 > wq0 + qpos);
-            if ((MASK != 0 && !MROW) || edge) {
+            if constexpr (MTILE) {
+                // the tile's own mask first (then the edge's, as without a mask)
+                if (mcls == kMaskTileBits) {
+#pragma unroll
+                    for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+                        for (int i = 0; i < 16; ++i)
+                            s[kb][i] = (mbits[kb] >> (8 * (i / 4) + (i % 4))) & 1u ? s[kb][i] : -INFINITY;
+                } else if (mcls == kMaskTileValues) {
+                    const float *mv = (const float *)a.mask + mtb * a.m_sb + (int64_t)min(lq, L - 1) * a.m_sl;
+#pragma unroll
+                    for (int kb = 0; kb < NKB; ++kb) {
+#pragma unroll
+                        for (int g = 0; g < 4; ++g) {
+                            const f32x4 x = *(const f32x4 *)(mv + min(k0 + 32 * kb + 8 * g + 4 * half, (S - 1) / 4 * 4));
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) s[kb][4 * g + e] = fmaf(x[e], inv_scale, s[kb][4 * g + e]);
+                        }
+                        __builtin_amdgcn_sched_barrier(0);  // 4 loads in flight: 16 would spill at head size 64
+                    }
+                }
+            }
+            if ((MASK != 0 && !MROW && !MTILE) || edge) {
                 // key k0 + 4half + c (c = 32kb + 8(i/4) + i%4, a constant per entry) is visible
                 // to this lane's row when c <= vis: one compare per score
                 const int vis = min(nkv - 1, CAUSAL ? lq + qpos : nkv - 1) - (k0 + 4 * half);
@@ -422,8 +490,8 @@ __global__ __launch_bounds__(64 * nw_of<D>(), DROP && (MASK == 1 || MASK == 2 ||
                     for (int i = 0; i < 16; ++i) {
                         const int key = k0 + 32 * kb + 8 * (i / 4) + 4 * half + (i % 4);
                         float x = s[kb][i];
-                        if constexpr (MROW) {
-                            // the mask row is already in s
+                        if constexpr (MROW || MTILE) {
+                            // the mask is already in s
                         } else if constexpr (MVEC) {
                             if constexpr (MBOOL) x = (mvb[kb][i / 4] >> (8 * (i % 4))) & 0xffu ? x : -INFINITY;
                             else x = fmaf(mvf[kb][i / 4][i % 4], inv_scale, x);
@@ -566,7 +634,7 @@ hipError_t launch_variant(const AttnFwdArgs &a, int nq, int order, int64_t grid,
 #define GT_PREFILL_LAUNCH_X(C, MK) \
     hipLaunchKernelGGL((prefill_fwd_kernel<T, D, C, MK, false, false, true>), dim3((unsigned)grid), dim3(64 * nw_of<D>()), 0, s, a, nq, order)
     if (a.dropout) {
-        if (a.rope_q) return hipErrorInvalidValue;  // dropout runs on unrotated queries only
+        if (a.rope_q || mode == 7) return hipErrorInvalidValue;  // dropout: unrotated queries, masks as given
         if (a.causal) {
             if (mode == 0) GT_PREFILL_LAUNCH_D(true, 0);
             else if (mode == 1) GT_PREFILL_LAUNCH_D(true, 1);
@@ -603,6 +671,7 @@ hipError_t launch_variant(const AttnFwdArgs &a, int nq, int order, int64_t grid,
                 else if (mode == 4) GT_PREFILL_LAUNCH_X(true, 4);
                 else if (mode == 5) GT_PREFILL_LAUNCH_X(true, 5);
                 else if (mode == 6) GT_PREFILL_LAUNCH_X(true, 6);
+                else if (mode == 7) GT_PREFILL_LAUNCH_X(true, 7);
                 else GT_PREFILL_LAUNCH_X(true, 2);
             } else {
                 if (mode == 0) GT_PREFILL_LAUNCH_X(false, 0);
@@ -610,6 +679,7 @@ hipError_t launch_variant(const AttnFwdArgs &a, int nq, int order, int64_t grid,
                 else if (mode == 4) GT_PREFILL_LAUNCH_X(false, 4);
                 else if (mode == 5) GT_PREFILL_LAUNCH_X(false, 5);
                 else if (mode == 6) GT_PREFILL_LAUNCH_X(false, 6);
+                else if (mode == 7) GT_PREFILL_LAUNCH_X(false, 7);
                 else GT_PREFILL_LAUNCH_X(false, 2);
             }
         }
@@ -619,6 +689,7 @@ hipError_t launch_variant(const AttnFwdArgs &a, int nq, int order, int64_t grid,
         else if (mode == 4) GT_PREFILL_LAUNCH(true, 4);
         else if (mode == 5) GT_PREFILL_LAUNCH(true, 5);
         else if (mode == 6) GT_PREFILL_LAUNCH(true, 6);
+        else if (mode == 7) GT_PREFILL_LAUNCH(true, 7);
         else GT_PREFILL_LAUNCH(true, 2);
     } else {
         if (mode == 0) GT_PREFILL_LAUNCH(false, 0);
@@ -626,6 +697,7 @@ hipError_t launch_variant(const AttnFwdArgs &a, int nq, int order, int64_t grid,
         else if (mode == 4) GT_PREFILL_LAUNCH(false, 4);
         else if (mode == 5) GT_PREFILL_LAUNCH(false, 5);
         else if (mode == 6) GT_PREFILL_LAUNCH(false, 6);
+        else if (mode == 7) GT_PREFILL_LAUNCH(false, 7);
         else GT_PREFILL_LAUNCH(false, 2);
     }
 #undef GT_PREFILL_LAUNCH
@@ -1176,6 +1248,8 @@ hipError_t launch_prefill_f32(const AttnFwdArgs &a, hipStream_t s) {
 }
 
 }  // namespace
+
+int attn_prefill_key_tile(const AttnFwdArgs &f) { return f.D == 64 ? bn_of<64>() : bn_of<128>(); }
 
 bool attn_prefill_f32_split(const AttnFwdArgs &f, int cd) {
     return cd == GT_F32 && prefill_f32_supported(f) && prefill_f32_split(f);

@@ -167,6 +167,66 @@ bool stage_mask(const gt_tensor *mask, int dev, int cd, AttnFwdArgs &a, Temps &t
     return true;
 }
 
+// The mask of a half-precision forward as tile classes (attn_mask_tiles.hip): one that varies along
+// the query rows and is shared by the heads, on the device in bool, float16, bfloat16 or float32.  The
+// pass over the mask and the list at the start of each workgroup cost about 8 us together, and a tile's
+// mask work saved about 1 us of a workgroup's walk, so the line is a number of key tiles: 8 for bool and
+// float32 masks (band, GPU time with the mask as given against tile classes: D64 B2 H16 L128 S512 18.2
+// against 21.7 us, S1024 33.0 against 28.5; D128 B4 H32 L256 S512 27.3 against 25.7, S1024 47.1 against
+// 37.3), 4 for half-precision ones, which are converted to float32 in a pass of their own otherwise (D64
+// B2 H16 L128 S384 20.1 against 20.4, S512 23.9 against 22.2; D128 B4 H32 L256 S256 21.6 against 19.8,
+// S1024 54.8 against 37.9).  float32 masks need the 4-key alignment of mode 6 (tiles with other values
+// than 0 and -inf are read in place).  Call with q, k, v and the options of `a` final.
+// 1: staged, 0: not of this kind, -1: error.
+int stage_mask_tiles(const gt_tensor *mask, int dev, int cd, AttnFwdArgs &a, gt_scratch &mem) {
+    if (!mask || (cd != GT_F16 && cd != GT_BF16) || a.dropout || a.rope_q || a.L <= 1 || a.S < 4) return 0;
+    const int kind = mask->dtype == GT_BOOL ? 0 : mask->dtype == GT_F16 ? 1 : mask->dtype == GT_BF16 ? 2 : mask->dtype == GT_F32 ? 3 : -1;
+    if (kind < 0 || mask->device_type != GT_DEV_CUDA || mask->device_index != dev) return 0;
+    const int n = mask->ndim;
+    const bool plane = mask->shape[n - 2] == a.L && mask->shape[n - 1] == a.S && (n == 2 || mask->shape[1] == 1);
+    const int64_t batches = n == 4 ? mask->shape[0] : 1;
+    if (!plane || a.B * a.H < 4 * batches) return 0;
+    const int64_t sb = n == 4 && batches > 1 ? mask->strides[0] : 0, sl = mask->strides[n - 2], ss = mask->strides[n - 1];
+    if (kind == 3) {
+        AttnFwdArgs probe = a;
+        probe.mask = gt_data(mask);
+        probe.mask_bool = 0;
+        probe.m_sb = sb;
+        probe.m_sh = 0;
+        probe.m_sl = sl;
+        probe.m_ss = ss;
+        if (attn_mask_mode(probe) != 6) return 0;
+    }
+    if (!attn_prefill_supported(a, cd)) return 0;
+    const int bn = attn_prefill_key_tile(a);
+    const int64_t nkt = (a.S + bn - 1) / bn, nqt = (a.L + kMaskTileRows - 1) / kMaskTileRows, words = (a.S + 31) / 32;
+    if (nkt < (kind == 1 || kind == 2 ? 4 : 8) || nkt > kMaskTilesMax || nqt > 65535 || batches > 65535) return 0;
+    const int64_t pitch = attn_mask_copy_pitch(a.S);
+    const size_t bits = ((size_t)(batches * a.L * words) * 4 + 255) / 256 * 256;
+    const size_t cls = ((size_t)(batches * nqt * nkt) + 255) / 256 * 256;
+    const size_t copy = kind == 1 || kind == 2 ? (size_t)(batches * a.L * pitch) * sizeof(float) : 0;
+    if (!gt_scratch_alloc(mem, bits + cls + copy, dev)) return -1;
+    char *p = (char *)mem.ptr();
+    AttnMaskTiles t{};
+    t.bits = (const uint32_t *)p;
+    t.cls = (const uint8_t *)(p + bits);
+    t.nkt = (int)nkt;
+    t.words = (int)words;
+    t.batched = batches > 1;
+    float *values = (float *)(p + bits + cls);
+    if (!gt_hip_check(launch_attn_mask_tiles(kind, gt_data(mask), batches, sb, sl, ss, a.L, a.S, bn, t, values, gt_stream()),
+                      "flash_attention: mask tiles kernel"))
+        return -1;
+    a.mt = t;
+    a.mask = copy ? (const void *)values : gt_data(mask);
+    a.mask_bool = kind == 0;
+    a.m_sb = copy ? a.L * pitch : sb;
+    a.m_sh = 0;
+    a.m_sl = copy ? pitch : sl;
+    a.m_ss = 1;
+    return 1;
+}
+
 void fill_qkv(AttnFwdArgs &a, const gt_tensor *q, const gt_tensor *k, const gt_tensor *v) {
     a.q = gt_data(q);
     a.k = gt_data(k);
@@ -443,11 +503,9 @@ int attention_forward(const char *who, const gt_tensor *q, const gt_tensor *k, c
         if (vs && vs->device_type != GT_DEV_CUDA) vs = stage(vs, dev, cd, tmp);
         ok = qs && ks && vs;
         AttnFwdArgs a{};
+        gt_scratch mtiles;
         if (ok) {
             fill_qkv(a, qs, ks, vs);
-            ok = stage_mask(mask, dev, cd, a, tmp);
-        }
-        if (ok) {
             a.o = gt_data(o);
             a.lse = lse ? gt_data(lse) : nullptr;
             a.o32 = o32 ? gt_data(o32) : nullptr;
@@ -470,6 +528,11 @@ int attention_forward(const char *who, const gt_tensor *q, const gt_tensor *k, c
                     a.o = const_cast<void *>(gt_data(po));
                     a.o32 = po32 ? const_cast<void *>(gt_data(po32)) : nullptr;
                 }
+            }
+            if (ok) {
+                // (fused RoPE takes masks as given)
+                const int tiled = qrope ? 0 : stage_mask_tiles(mask, dev, cd, a, mtiles);
+                ok = tiled > 0 || (tiled == 0 && stage_mask(mask, dev, cd, a, tmp));
             }
             if (qrope) {
                 a.rope_q = qrope->table;
