@@ -325,8 +325,7 @@ gt_tensor *deliver(gt_tensor *dev_t, bool to_host) { return gt_deliver(dev_t, to
 // Returns 1 when it ran, 0 when the shapes do not suit the kernel (the caller then dequantizes), -1
 // on error.
 int run_q8_decode(const gt_tensor *q, const gt_tensor *k, const gt_tensor *v, const gt_tensor *mask, float scale,
-                  int is_causal, int dev, gt_tensor *o, gt_tensor *lse, Temps &tmp, const int32_t *kv_len = nullptr,
-                  const int32_t *q_pos = nullptr) {
+                  int is_causal, int dev, gt_tensor *o, gt_tensor *lse, Temps &tmp, const int32_t *kv_len = nullptr) {
     const int qd = q->dtype;
     const gt_tensor *qs = stage(q, dev, qd, tmp);
     const gt_tensor *ks = k->device_type == GT_DEV_CUDA && k->device_index == dev ? k : tmp.keep(gt_to_device_dense(k, dev, -1));
@@ -340,7 +339,7 @@ int run_q8_decode(const gt_tensor *q, const gt_tensor *k, const gt_tensor *v, co
     a.causal = is_causal ? 1 : 0;
     a.out_dtype = qd;
     a.kv_len = kv_len;
-    a.q_pos = q_pos;
+    a.q_tail = kv_len != nullptr;  // (a KV cache: the query is its last token)
     if (!attn_decode_q8_supported(a, qd)) return 0;
     if (!stage_mask(mask, dev, qd, a, tmp)) return -1;
     DecodeArgs da{};
@@ -1312,18 +1311,12 @@ struct gt_kv_cache {
     int dev = 0;
     gt_tensor *k = nullptr, *v = nullptr;  // (B, Hkv, cap, D), zero-filled at creation
     std::vector<int32_t> len;              // tokens held per sequence (the authoritative copy)
-    gt_tensor *len_dev = nullptr;          // device copy of len (int32, B)
-    gt_tensor *pos_dev = nullptr;          // position of query row 0 per sequence (int32, B)
+    // device copy of len (int32, B), and the array that the next append writes the new lengths to (its
+    // workgroups still read the old ones); the two swap, so nothing is uploaded
+    gt_tensor *len_dev = nullptr, *len_next = nullptr;
 };
 
 namespace {
-
-bool kv_upload(gt_tensor *dst, const std::vector<int32_t> &src) {
-    // pageable source: returns once the bytes are staged, so `src` may change afterwards
-    return gt_hip_check(hipMemcpyAsync(gt_data(dst), src.data(), src.size() * sizeof(int32_t), hipMemcpyHostToDevice,
-                                       gt_stream()),
-                        "kv cache: length upload");
-}
 
 bool kv_zero(gt_tensor *t) {
     return gt_hip_check(gt_launch_fill_zero(gt_data(t), (int64_t)gt_dtype_nbytes(t->dtype, t->numel), gt_stream()),
@@ -1394,10 +1387,9 @@ extern "C" gt_kv_cache *gt_kv_cache_create(int64_t batch, int64_t n_head_kv, int
     c->k = gt_new_tensor(4, sh, dtype, GT_DEV_CUDA, device_index);
     c->v = c->k ? gt_new_tensor(4, sh, dtype, GT_DEV_CUDA, device_index) : nullptr;
     c->len_dev = c->v ? gt_new_tensor(1, lsh, GT_I32, GT_DEV_CUDA, device_index) : nullptr;
-    c->pos_dev = c->len_dev ? gt_new_tensor(1, lsh, GT_I32, GT_DEV_CUDA, device_index) : nullptr;
+    c->len_next = c->len_dev ? gt_new_tensor(1, lsh, GT_I32, GT_DEV_CUDA, device_index) : nullptr;
     // rows past a sequence's length are read (and weighted 0) by the kernels: keep them finite
-    if (!c->pos_dev || !kv_zero(c->k) || !kv_zero(c->v) || !kv_upload(c->len_dev, c->len) ||
-        !kv_upload(c->pos_dev, c->len)) {
+    if (!c->len_next || !kv_zero(c->k) || !kv_zero(c->v) || !kv_zero(c->len_dev)) {
         gt_kv_cache_free(c);
         return nullptr;
     }
@@ -1409,7 +1401,7 @@ extern "C" void gt_kv_cache_free(gt_kv_cache *c) {
     gt_tensor_free(c->k);
     gt_tensor_free(c->v);
     gt_tensor_free(c->len_dev);
-    gt_tensor_free(c->pos_dev);
+    gt_tensor_free(c->len_next);
     delete c;
 }
 
@@ -1423,9 +1415,15 @@ extern "C" int gt_kv_cache_clear(gt_kv_cache *c, int64_t seq) {
                      " sequences");
         return -1;
     }
+    if (!gt_device_ok(c->dev)) return -1;
+    int32_t *len = (int32_t *)gt_data(c->len_dev);
     if (seq < 0) std::fill(c->len.begin(), c->len.end(), 0);
     else c->len[(size_t)seq] = 0;
-    return kv_upload(c->len_dev, c->len) ? 0 : -1;
+    return gt_hip_check(gt_launch_fill_zero(seq < 0 ? len : len + seq, (seq < 0 ? c->B : 1) * (int64_t)sizeof(int32_t),
+                                            gt_stream()),
+                        "kv cache clear kernel")
+               ? 0
+               : -1;
 }
 
 extern "C" int64_t gt_kv_cache_length(const gt_kv_cache *c, int64_t seq) {
@@ -1496,11 +1494,21 @@ int kv_append(const char *who, gt_kv_cache *c, const gt_tensor *k, const gt_tens
         }
     }
     if (!gt_device_ok(c->dev)) return -1;
+    if (T == 0) return 0;
     Temps tmp;
     const int32_t *pos = (const int32_t *)gt_data(c->len_dev);
+    int32_t *next = (int32_t *)gt_data(c->len_next);
     gt_scratch table;
+    // keys and values of one half or float32 dtype in aligned rows: one launch, which also forms the
+    // angles of a few rows and the lengths after it
+    const bool on_dev = k->device_type == GT_DEV_CUDA && k->device_index == c->dev && v->device_type == GT_DEV_CUDA &&
+                        v->device_index == c->dev;
+    const int n_dims = rope ? rope->n_dims : 0;
+    const bool pair = on_dev && k->dtype == v->dtype && k->dtype != GT_Q8_0 &&
+                      gt_kv_append_vec_ok(gt_data(k), k->dtype, k->strides, gt_data(c->k), c->dtype, c->Hkv, T, c->D, n_dims) &&
+                      gt_kv_append_vec_ok(gt_data(v), v->dtype, v->strides, gt_data(c->v), c->dtype, c->Hkv, T, c->D, 0);
     gt_rope_apply ra{};
-    if (rope && T > 0) {
+    if (rope && !(pair && gt_kv_rope_inline(c->B, c->Hkv, T, c->D))) {
         // (cos, sin) of table row b * T + t at position len[b] + t
         if (!gt_scratch_alloc(table, (size_t)(c->B * T) * (size_t)(rope->n_dims / 2) * 2 * sizeof(float), c->dev) ||
             !gt_hip_check(gt_launch_rope_table(nullptr, pos, T, c->B * T, rope->n_dims,
@@ -1512,7 +1520,15 @@ int kv_append(const char *who, gt_kv_cache *c, const gt_tensor *k, const gt_tens
         ra.n_dims = rope->n_dims;
         ra.neox = rope->mode == 2;
     }
-    for (const gt_tensor *src : {k, v}) {
+    if (pair) {
+        gt_kv_rope kr{};
+        if (rope) kr = {table.ptr(), rope->n_dims, rope->mode == 2, gt_rope_theta_scale(rope->freq_base, rope->n_dims), rope->freq_scale};
+        if (!gt_hip_check(gt_launch_kv_append_pair(gt_data(k), gt_data(v), k->dtype, k->strides, v->strides, gt_data(c->k),
+                                                   gt_data(c->v), c->dtype, pos, next, c->B, c->Hkv, T, c->D, c->cap,
+                                                   rope ? &kr : nullptr, gt_stream()),
+                          "kv cache append kernel"))
+            return -1;
+    } else for (const gt_tensor *src : {k, v}) {
         const bool rotate = rope && src == k;
         const gt_tensor *s = src->device_type == GT_DEV_CUDA && src->device_index == c->dev
                                  ? src
@@ -1528,11 +1544,13 @@ int kv_append(const char *who, gt_kv_cache *c, const gt_tensor *k, const gt_tens
             s->dtype == GT_Q8_0
                 ? gt_launch_kv_append_blocks(gt_data(s), gt_data(dst), pos, c->B, c->Hkv, T, c->D, c->cap, gt_stream())
                 : gt_launch_kv_append(gt_data(s), s->dtype, s->strides, gt_data(dst), c->dtype, pos, c->B, c->Hkv, T,
-                                      c->D, c->cap, rotate && T > 0 ? &ra : nullptr, gt_stream());
+                                      c->D, c->cap, rotate ? &ra : nullptr, gt_stream());
         if (!gt_hip_check(e, "kv cache append kernel")) return -1;
     }
+    if (!pair && !gt_hip_check(gt_launch_kv_advance(pos, next, T, c->B, gt_stream()), "kv cache lengths kernel")) return -1;
+    std::swap(c->len_dev, c->len_next);
     for (auto &n : c->len) n += (int32_t)T;
-    return kv_upload(c->len_dev, c->len) ? 0 : -1;
+    return 0;
 }
 
 }  // namespace
@@ -1565,7 +1583,6 @@ extern "C" gt_tensor *gt_kv_cache_attention(gt_kv_cache *c, const gt_tensor *q, 
     }
     const int64_t B = c->B, H = q->shape[1], L = q->shape[2], D = c->D;
     // query row l of sequence b is token len[b] - L + l
-    std::vector<int32_t> pos((size_t)B);
     int64_t maxlen = 0;
     for (int64_t b = 0; b < B; ++b) {
         const int64_t n = c->len[(size_t)b];
@@ -1574,13 +1591,12 @@ extern "C" gt_tensor *gt_kv_cache_attention(gt_kv_cache *c, const gt_tensor *q, 
                          " tokens, fewer than the " + std::to_string(L) + " query rows (append them first)");
             return nullptr;
         }
-        pos[(size_t)b] = (int32_t)(n - L);
         maxlen = std::max<int64_t>(maxlen, n);
     }
     if (scale <= 0.0f) scale = 1.0f / std::sqrt((float)D);
     const int dev = c->dev;
-    if (!gt_device_ok(dev) || !kv_upload(c->pos_dev, pos)) return nullptr;
-    const int32_t *kv_len = (const int32_t *)gt_data(c->len_dev), *q_pos = (const int32_t *)gt_data(c->pos_dev);
+    if (!gt_device_ok(dev)) return nullptr;
+    const int32_t *kv_len = (const int32_t *)gt_data(c->len_dev);
     const bool host_io = q->device_type != GT_DEV_CUDA;
     const int64_t osh[4] = {B, H, L, D};
     gt_tensor *o = gt_new_tensor(4, osh, q->dtype, GT_DEV_CUDA, dev);
@@ -1589,7 +1605,7 @@ extern "C" gt_tensor *gt_kv_cache_attention(gt_kv_cache *c, const gt_tensor *q, 
     bool ok = true;
     int q8 = 0;
     if (o->numel > 0 && c->dtype == GT_Q8_0 && q->dtype != GT_F64 && L == 1) {
-        q8 = run_q8_decode(q, c->k, c->v, nullptr, scale, is_causal, dev, o, nullptr, tmp, kv_len, q_pos);
+        q8 = run_q8_decode(q, c->k, c->v, nullptr, scale, is_causal, dev, o, nullptr, tmp, kv_len);
         ok = q8 >= 0;
     }
     if (ok && q8 == 0 && o->numel > 0) {
@@ -1646,7 +1662,7 @@ extern "C" gt_tensor *gt_kv_cache_attention(gt_kv_cache *c, const gt_tensor *q, 
             a.causal = is_causal ? 1 : 0;
             a.out_dtype = q->dtype;
             a.kv_len = kv_len;
-            a.q_pos = q_pos;
+            a.q_tail = 1;
             ok = dispatch_forward(a, cd, dev);
             if (ok && po) ok = unpad_heads(po, o);
         }

@@ -316,16 +316,47 @@ __device__ inline void load8(const void *base, int64_t e0, float *v) {
 // kv_append_kernel: the rotation in float32 rounded to the source dtype, then the cache dtype;
 // a Q8_0 cache quantizes with four threads per block (the block's |x| max by two lane
 // exchanges) and the operations of q8_0_quantize_lane.
+// blockIdx.y picks one of up to two tensors (keys and values), of which the first is rotated; with
+// pos_next, the first workgroup writes the lengths after the append.
+struct KvAppendVec {
+    const void *src[2];
+    void *dst[2];
+    int64_t st[2][3];
+    const int32_t *pos;
+    int32_t *pos_next;  // not pos: every workgroup reads that
+    int B, Hkv, T, D;
+    int64_t cap, n8;
+    const float2 *table;
+    int n_dims, neox;  // n_dims 0: no rotation
+    float theta_scale, freq_scale;
+};
 template <int SDT, int DDT>
-__global__ __launch_bounds__(256) void kv_append_vec_kernel(const void *__restrict__ src, int64_t s_sb, int64_t s_sh,
-                                                            int64_t s_st, void *__restrict__ dst,
-                                                            const int32_t *__restrict__ pos, int Hkv, int T, int D,
-                                                            int64_t cap, int64_t n8, const float2 *__restrict__ rope_table,
-                                                            int n_dims, int neox) {
+__global__ __launch_bounds__(256) void kv_append_vec_kernel(KvAppendVec a) {
+    const void *__restrict__ src = a.src[blockIdx.y];
+    void *__restrict__ dst = a.dst[blockIdx.y];
+    const int32_t *__restrict__ pos = a.pos;
+    const int64_t s_sb = a.st[blockIdx.y][0], s_sh = a.st[blockIdx.y][1], s_st = a.st[blockIdx.y][2];
+    const int Hkv = a.Hkv, T = a.T, D = a.D, n_dims = blockIdx.y == 0 ? a.n_dims : 0, neox = a.neox;
+    const int64_t cap = a.cap, n8 = a.n8;
+    if (a.pos_next && blockIdx.x == 0 && blockIdx.y == 0)
+        for (int b = threadIdx.x; b < a.B; b += 256) a.pos_next[b] = pos[b] + T;
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const bool live = i < n8;
     const int64_t ic = live ? i : 0;
     const int per = D / 8;
+    __shared__ float2 s_cs[kRopeInlineEntries];
+    const int64_t r0 = (int64_t)blockIdx.x * 256 / per;  // the workgroup's first row
+    if (n_dims && !a.table) {
+        // the rows' angles: one set per sequence for a single token, else one per row
+        const int half = n_dims / 2;
+        const int64_t rl = min((int64_t)blockIdx.x * 256 + 255, n8 - 1) / per;
+        const int n = (int)(T == 1 ? rl / Hkv - r0 / Hkv + 1 : rl - r0 + 1) * half;
+        for (int e = threadIdx.x; e < n; e += 256) {
+            const int64_t rr = T == 1 ? (r0 / Hkv + e / half) * Hkv : r0 + e / half;
+            s_cs[e] = rope_cos_sin(rope_theta(pos[rr / T / Hkv] + (int)(rr % T), e % half, a.theta_scale), a.freq_scale);
+        }
+        __syncthreads();
+    }
     const int j = (int)(ic % per);
     const int64_t r = ic / per;  // source row (b, h, t)
     const int t = (int)(r % T);
@@ -336,19 +367,25 @@ __global__ __launch_bounds__(256) void kv_append_vec_kernel(const void *__restri
     const int64_t srow = b * s_sb + h * s_sh + (int64_t)t * s_st;
     float v[8];
     load8<SDT>(src, srow + d0, v);
-    if (rope_table && d0 < n_dims) {
+    if (d0 < n_dims) {
         const int half = n_dims / 2;
         const bool lo_chunk = d0 < half;  // NeoX: the whole chunk is on one side of half
         float w[8];
         if (neox) load8<SDT>(src, srow + (lo_chunk ? d0 + half : d0 - half), w);
+        // the chunk's pairs in order: first, first + 1, ...
+        const int first = neox ? (lo_chunk ? d0 : d0 - half) : d0 >> 1, np = neox ? 8 : 4;
+        float2 cs8[8];
+        const float2 *tab = a.table ? a.table + ((int64_t)b * T + t) * half
+                                    : s_cs + (int)(T == 1 ? bh / Hkv - r0 / Hkv : r - r0) * half;
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            if (e < np) cs8[e] = tab[first + e];
         float rr[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-            const int d = d0 + e;
             const bool lo = neox ? lo_chunk : (e & 1) == 0;
             const float other = neox ? w[e] : v[e ^ 1];
-            const int pair = neox ? (lo ? d : d - half) : (d >> 1);
-            const float2 cs = rope_table[((int64_t)b * T + t) * half + pair];
+            const float2 cs = neox ? cs8[e] : cs8[e >> 1];
             float x = lo ? rope_rot_lo(v[e], other, cs) : rope_rot_hi(other, v[e], cs);
             if constexpr (SDT == GT_F16) x = d_f16_to_f32(d_f32_to_f16(x));
             else if constexpr (SDT == GT_BF16) x = u2f((uint32_t)d_f32_to_bf16(x) << 16);
@@ -394,6 +431,11 @@ __global__ __launch_bounds__(256) void kv_append_vec_kernel(const void *__restri
             *(uint4 *)((uint16_t *)dst + o) = make_uint4(w[0], w[1], w[2], w[3]);
         }
     }
+}
+
+__global__ void kv_advance_kernel(const int32_t *__restrict__ pos, int32_t *__restrict__ next, int32_t T, int B) {
+    const int b = blockIdx.x * 256 + threadIdx.x;
+    if (b < B) next[b] = pos[b] + T;
 }
 
 // KV-cache append of rows that are already Q8_0: row (b, h, t) of the dense Q8_0 src
@@ -617,20 +659,76 @@ hipError_t gt_launch_fill_zero(void *p, int64_t bytes, hipStream_t stream) {
 }
 
 template <int SDT>
-hipError_t launch_kv_append_vec(const void *src, const int64_t *st, void *dst, int ddt, const int32_t *pos, int64_t Hkv,
-                                int64_t T, int64_t D, int64_t cap, int64_t n8, const gt_rope_apply *rope,
-                                hipStream_t stream) {
-    const dim3 grid((unsigned)((n8 + 255) / 256));
-    const float2 *tab = rope ? (const float2 *)rope->table : nullptr;
-    const int nd = rope ? rope->n_dims : 0, nx = rope ? rope->neox : 0;
-#define GT_KV_APPEND_VEC(DDT)                                                                                          \
-    hipLaunchKernelGGL((kv_append_vec_kernel<SDT, DDT>), grid, dim3(256), 0, stream, src, st[0], st[1], st[2], dst, pos, \
-                       (int)Hkv, (int)T, (int)D, cap, n8, tab, nd, nx)
+hipError_t launch_kv_append_vec(const KvAppendVec &a, int ntensors, int ddt, hipStream_t stream) {
+    const dim3 grid((unsigned)((a.n8 + 255) / 256), (unsigned)ntensors);
+#define GT_KV_APPEND_VEC(DDT) hipLaunchKernelGGL((kv_append_vec_kernel<SDT, DDT>), grid, dim3(256), 0, stream, a)
     if (ddt == GT_F32) GT_KV_APPEND_VEC(GT_F32);
     else if (ddt == GT_F16) GT_KV_APPEND_VEC(GT_F16);
     else if (ddt == GT_BF16) GT_KV_APPEND_VEC(GT_BF16);
     else GT_KV_APPEND_VEC(GT_Q8_0);
 #undef GT_KV_APPEND_VEC
+    return hipGetLastError();
+}
+
+hipError_t launch_kv_append_vec(const KvAppendVec &a, int ntensors, int sdt, int ddt, hipStream_t stream) {
+    if (sdt == GT_F32) return launch_kv_append_vec<GT_F32>(a, ntensors, ddt, stream);
+    if (sdt == GT_F16) return launch_kv_append_vec<GT_F16>(a, ntensors, ddt, stream);
+    return launch_kv_append_vec<GT_BF16>(a, ntensors, ddt, stream);
+}
+
+bool gt_kv_append_vec_ok(const void *src, int src_dtype, const int64_t *src_strides, const void *dst, int dst_dtype,
+                         int64_t Hkv, int64_t T, int64_t D, int n_dims) {
+    // contiguous rows of a float32 / float16 / bfloat16 source starting 16-byte aligned
+    const int es = src_dtype == GT_F32 ? 4 : 2;
+    const bool vec_src = src_dtype == GT_F32 || src_dtype == GT_F16 || src_dtype == GT_BF16;
+    const bool vec_dst = dst_dtype == GT_F32 || dst_dtype == GT_F16 || dst_dtype == GT_BF16 || dst_dtype == GT_Q8_0;
+    return vec_src && vec_dst && src_strides[3] == 1 && D % 8 == 0 && (uintptr_t)src % 16 == 0 &&
+           (src_strides[0] * es) % 16 == 0 && (src_strides[1] * es) % 16 == 0 && (src_strides[2] * es) % 16 == 0 &&
+           (uintptr_t)dst % 16 == 0 && n_dims % 16 == 0 && T < (1LL << 31) && D < (1LL << 31) && Hkv < (1LL << 31) &&
+           (dst_dtype != GT_Q8_0 || D % 32 == 0);
+}
+
+bool gt_kv_rope_inline(int64_t B, int64_t Hkv, int64_t T, int64_t D) {
+    return D <= kRopeInlineMaxDim && B * Hkv * T * (D / 8) <= kRopeInlineThreads;
+}
+
+hipError_t gt_launch_kv_append_pair(const void *k, const void *v, int src_dtype, const int64_t *k_strides,
+                                    const int64_t *v_strides, void *kdst, void *vdst, int dst_dtype, const int32_t *pos,
+                                    int32_t *pos_next, int64_t B, int64_t Hkv, int64_t T, int64_t D, int64_t cap,
+                                    const gt_kv_rope *rope, hipStream_t stream) {
+    const int64_t n8 = B * Hkv * T * D / 8;
+    if (n8 <= 0 || (n8 + 255) / 256 > 0x7fffffffLL || B > 0x7fffffffLL) return hipErrorInvalidConfiguration;
+    if (rope && (rope->n_dims < 2 || rope->n_dims > D)) return hipErrorInvalidValue;
+    KvAppendVec a{};
+    a.src[0] = k;
+    a.src[1] = v;
+    a.dst[0] = kdst;
+    a.dst[1] = vdst;
+    for (int i = 0; i < 3; ++i) {
+        a.st[0][i] = k_strides[i];
+        a.st[1][i] = v_strides[i];
+    }
+    a.pos = pos;
+    a.pos_next = pos_next;
+    a.B = (int)B;
+    a.Hkv = (int)Hkv;
+    a.T = (int)T;
+    a.D = (int)D;
+    a.cap = cap;
+    a.n8 = n8;
+    if (rope) {
+        a.table = (const float2 *)rope->table;
+        a.n_dims = rope->n_dims;
+        a.neox = rope->neox;
+        a.theta_scale = rope->theta_scale;
+        a.freq_scale = rope->freq_scale;
+    }
+    return launch_kv_append_vec(a, 2, src_dtype, dst_dtype, stream);
+}
+
+hipError_t gt_launch_kv_advance(const int32_t *pos, int32_t *pos_next, int64_t T, int64_t B, hipStream_t stream) {
+    hipLaunchKernelGGL(kv_advance_kernel, dim3((unsigned)((B + 255) / 256)), dim3(256), 0, stream, pos, pos_next, (int32_t)T,
+                       (int)B);
     return hipGetLastError();
 }
 
@@ -642,19 +740,24 @@ hipError_t gt_launch_kv_append(const void *src, int src_dtype, const int64_t *sr
     const int64_t blocks = (n + 255) / 256;
     if (blocks > 0x7fffffffLL) return hipErrorInvalidConfiguration;
     if (rope && (rope->n_dims < 2 || rope->n_dims % 2 != 0 || rope->n_dims > D)) return hipErrorInvalidValue;
-    // fast path: contiguous rows of a float32 / float16 / bfloat16 source starting 16-byte aligned
-    const int es = src_dtype == GT_F32 ? 4 : 2;
-    const bool vec_src = src_dtype == GT_F32 || src_dtype == GT_F16 || src_dtype == GT_BF16;
-    const bool vec_dst = dst_dtype == GT_F32 || dst_dtype == GT_F16 || dst_dtype == GT_BF16 || dst_dtype == GT_Q8_0;
-    if (vec_src && vec_dst && src_strides[3] == 1 && D % 8 == 0 && (uintptr_t)src % 16 == 0 &&
-        (src_strides[0] * es) % 16 == 0 && (src_strides[1] * es) % 16 == 0 && (src_strides[2] * es) % 16 == 0 &&
-        (uintptr_t)dst % 16 == 0 && (!rope || rope->n_dims % 16 == 0) && T < (1LL << 31) && D < (1LL << 31) &&
-        Hkv < (1LL << 31) && (dst_dtype != GT_Q8_0 || D % 32 == 0)) {
-        const int64_t n8 = n / 8;
-        if ((n8 + 255) / 256 > 0x7fffffffLL) return hipErrorInvalidConfiguration;
-        if (src_dtype == GT_F32) return launch_kv_append_vec<GT_F32>(src, src_strides, dst, dst_dtype, pos, Hkv, T, D, cap, n8, rope, stream);
-        if (src_dtype == GT_F16) return launch_kv_append_vec<GT_F16>(src, src_strides, dst, dst_dtype, pos, Hkv, T, D, cap, n8, rope, stream);
-        return launch_kv_append_vec<GT_BF16>(src, src_strides, dst, dst_dtype, pos, Hkv, T, D, cap, n8, rope, stream);
+    if (gt_kv_append_vec_ok(src, src_dtype, src_strides, dst, dst_dtype, Hkv, T, D, rope ? rope->n_dims : 0)) {
+        KvAppendVec a{};
+        a.src[0] = src;
+        a.dst[0] = dst;
+        for (int i = 0; i < 3; ++i) a.st[0][i] = src_strides[i];
+        a.pos = pos;
+        a.Hkv = (int)Hkv;
+        a.T = (int)T;
+        a.D = (int)D;
+        a.cap = cap;
+        a.n8 = n / 8;
+        if ((a.n8 + 255) / 256 > 0x7fffffffLL) return hipErrorInvalidConfiguration;
+        if (rope) {
+            a.table = (const float2 *)rope->table;
+            a.n_dims = rope->n_dims;
+            a.neox = rope->neox;
+        }
+        return launch_kv_append_vec(a, 1, src_dtype, dst_dtype, stream);
     }
     hipLaunchKernelGGL(kv_append_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, src, src_dtype, src_strides[0],
                        src_strides[1], src_strides[2], src_strides[3], dst, dst_dtype, pos, Hkv, T, D, cap, n,

@@ -127,6 +127,25 @@ struct gt_rope_apply {
 hipError_t gt_launch_kv_append(const void *src, int src_dtype, const int64_t *src_strides, void *dst, int dst_dtype,
                                const int32_t *pos, int64_t B, int64_t Hkv, int64_t T, int64_t D, int64_t cap,
                                const gt_rope_apply *rope, hipStream_t stream);
+// The keys and values of one append in one launch, and the lengths after it: `pos` (device int32 per
+// sequence) is read, pos[b] + T written to pos_next (another array).  Both sources of one dtype in
+// rows that the vector path takes (gt_kv_append_vec_ok); rope as above for the keys, with angles formed
+// in the kernel when `table` is null (theta_scale, freq_scale).
+struct gt_kv_rope {
+    const void *table;
+    int n_dims, neox;
+    float theta_scale, freq_scale;
+};
+bool gt_kv_append_vec_ok(const void *src, int src_dtype, const int64_t *src_strides, const void *dst, int dst_dtype,
+                         int64_t Hkv, int64_t T, int64_t D, int n_dims);
+hipError_t gt_launch_kv_append_pair(const void *k, const void *v, int src_dtype, const int64_t *k_strides,
+                                    const int64_t *v_strides, void *kdst, void *vdst, int dst_dtype, const int32_t *pos,
+                                    int32_t *pos_next, int64_t B, int64_t Hkv, int64_t T, int64_t D, int64_t cap,
+                                    const gt_kv_rope *rope, hipStream_t stream);
+// Whether an append of these rows forms its RoPE angles in the kernel.
+bool gt_kv_rope_inline(int64_t B, int64_t Hkv, int64_t T, int64_t D);
+// pos_next[b] = pos[b] + T for b < B.
+hipError_t gt_launch_kv_advance(const int32_t *pos, int32_t *pos_next, int64_t T, int64_t B, hipStream_t stream);
 // KV-cache append of Q8_0 rows: the dense Q8_0 src (B, Hkv, T, D), D % 32 == 0, copied block by
 // block (bytes unchanged) to rows pos[b] + t of the Q8_0 cache (B, Hkv, cap, D).
 hipError_t gt_launch_kv_append_blocks(const void *src, void *dst, const int32_t *pos, int64_t B, int64_t Hkv,
@@ -137,9 +156,17 @@ hipError_t gt_launch_rope_table(const int32_t *pos, const int32_t *base, int64_t
                                 float theta_scale, float freq_scale, int backward, void *table, hipStream_t stream);
 // RoPE rotation of x (B, H, S, D; element strides) into the dense y of the same float dtype, with
 // the angles of table row b * table_b_stride + s; mode 0 NORMAL, 2 NEOX.
+// Without a table (null): with the angles of position angles->pos[s], formed in the kernel
+// (gt_rope_inline: few enough elements, and rows short enough, for that).
+struct gt_rope_angles {
+    const int32_t *pos;
+    float theta_scale, freq_scale;
+    int backward;
+};
+bool gt_rope_inline(int64_t numel, int64_t D);
 hipError_t gt_launch_rope(const void *x, int dtype, const int64_t *strides, void *y, const void *table,
                           int64_t table_b_stride, int64_t B, int64_t H, int64_t S, int64_t D, int n_dims, int mode,
-                          hipStream_t stream);
+                          hipStream_t stream, const gt_rope_angles *angles = nullptr);
 // ---- RoPE argument checks (gt_rope_ops.cpp) ----------------------------------------------------
 // mode 0/2, even n_dims in [2, head_dim], positive finite freq_base, finite freq_scale; the
 // reference's messages prefixed with `who`.

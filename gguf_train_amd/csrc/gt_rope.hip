@@ -9,7 +9,8 @@
 //   i < n_dims/2; elements from n_dims on pass through.  y_lo = x_lo c - x_hi s,
 //   y_hi = x_lo s + x_hi c in float32, on inputs converted to float32, rounded to the output type.
 //
-// Two kernels: the angle table (one (cos, sin) pair per position and pair index, computed once per
+// Few rows (kRopeInlineThreads): one kernel, each thread forming its own angles.  Otherwise two
+// kernels: the angle table (one (cos, sin) pair per position and pair index, computed once per
 // call and shared by every head), then the rotation, which is HBM-bound element work: one thread
 // per VEC consecutive elements of a row (16-byte loads and stores for dense rows); a NeoX thread
 // also loads its partner group from the other half of the same row, cache lines the neighbouring
@@ -26,7 +27,9 @@ struct RopeArgs {
     const void *x;
     int64_t sb, sh, ss, sd;   // element strides of x (B, H, S, D)
     void *y;                  // dense (B, H, S, D) output
-    const float2 *table;      // (table row, pair) -> (cos, sin)
+    const float2 *table;      // (table row, pair) -> (cos, sin); null: from pos
+    const int32_t *pos;       // position of row s
+    float theta_scale, freq_scale, sin_sign;
     int64_t tb;               // table row of (b, s) = b * tb + s
     int64_t H, S, D;
     int n_dims, half, neox;
@@ -52,12 +55,8 @@ __global__ void rope_table_kernel(const int32_t *__restrict__ pos, const int32_t
     const int64_t r = idx / half;
     const int i = (int)(idx - r * half);
     const int32_t p = base ? base[r / T] + (int32_t)(r % T) : pos[r];
-    float theta = (float)p;
-    for (int j = 0; j < i; ++j) theta *= theta_scale;  // the same chain of float32 products as ggml
-    const float angle = freq_scale * theta;
-    float sn, cs;
-    sincosf(angle, &sn, &cs);
-    table[idx] = make_float2(cs, sin_sign * sn);
+    const float2 cs = rope_cos_sin(rope_theta(p, i, theta_scale), freq_scale);
+    table[idx] = make_float2(cs.x, sin_sign * cs.y);
 }
 
 template <typename T, int VEC>
@@ -74,18 +73,41 @@ __device__ inline void load_group(const T *row, int d, int64_t sd, float *v) {
     }
 }
 
-template <typename T, int VEC>
+// INLINE: the angles of a.pos instead of a.table.
+template <typename T, int VEC, bool INLINE>
 __global__ void __launch_bounds__(256) rope_kernel(RopeArgs a) {
     const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= a.ngroups) return;
     const int64_t gpr = a.D / VEC;
+    __shared__ float2 s_cs[INLINE ? kRopeInlineEntries : 1];
+    const int64_t row0 = (int64_t)blockIdx.x * 256 / gpr;  // the workgroup's first row
+    if constexpr (INLINE) {
+        // the rows' angles, once for all of them when they are at one position
+        const int64_t rowl = min((int64_t)blockIdx.x * 256 + 255, a.ngroups - 1) / gpr;
+        const int n = (a.S == 1 ? 1 : (int)(rowl - row0 + 1)) * a.half;
+        for (int e = threadIdx.x; e < n; e += 256) {
+            const int64_t s = (row0 + e / a.half) % a.S;
+            const float2 cs = rope_cos_sin(rope_theta(a.pos[s], e % a.half, a.theta_scale), a.freq_scale);
+            s_cs[e] = make_float2(cs.x, a.sin_sign * cs.y);
+        }
+        __syncthreads();
+    }
+    if (g >= a.ngroups) return;
     const int64_t row = g / gpr;
     const int d0 = (int)(g - row * gpr) * VEC;
     const int64_t s = row % a.S, bh = row / a.S, h = bh % a.H, b = bh / a.H;
     const T *xr = static_cast<const T *>(a.x) + b * a.sb + h * a.sh + s * a.ss;
-    const float2 *tab = a.table + (b * a.tb + s) * a.half;
     float v[VEC], o[VEC];
     load_group<T, VEC>(xr, d0, a.sd, v);
+    // the pairs of this group in order: first, first + 1, ...
+    const int first = a.neox ? (d0 < a.half ? d0 : d0 - a.half) : d0 >> 1;
+    float2 cs8[VEC];
+    if (d0 < a.n_dims) {
+        const int np = a.neox ? VEC : (VEC + 1) / 2;
+        const float2 *tab = INLINE ? s_cs + (a.S == 1 ? 0 : (int)(row - row0) * a.half) : a.table + (b * a.tb + s) * a.half;
+#pragma unroll
+        for (int j = 0; j < VEC; ++j)
+            if (j < np) cs8[j] = tab[first + j];
+    }
     if (d0 >= a.n_dims) {
 #pragma unroll
         for (int j = 0; j < VEC; ++j) o[j] = v[j];
@@ -94,12 +116,12 @@ __global__ void __launch_bounds__(256) rope_kernel(RopeArgs a) {
             // the pair (d0 & ~1, d0 | 1); n_dims is even, so both are rotated
             float w;
             load_group<T, 1>(xr, d0 ^ 1, a.sd, &w);
-            const float2 cs = tab[d0 >> 1];
+            const float2 cs = cs8[0];
             o[0] = (d0 & 1) ? rope_rot_hi(w, v[0], cs) : rope_rot_lo(v[0], w, cs);
         } else {
 #pragma unroll
             for (int j = 0; j < VEC; j += 2) {
-                const float2 cs = tab[(d0 + j) >> 1];
+                const float2 cs = cs8[j >> 1];
                 o[j] = rope_rot_lo(v[j], v[j + 1], cs);
                 o[j + 1] = rope_rot_hi(v[j], v[j + 1], cs);
             }
@@ -109,10 +131,9 @@ __global__ void __launch_bounds__(256) rope_kernel(RopeArgs a) {
         const int pd = lo ? d0 + a.half : d0 - a.half;
         float w[VEC];
         load_group<T, VEC>(xr, pd, a.sd, w);
-        const int i0 = lo ? d0 : pd;
 #pragma unroll
         for (int j = 0; j < VEC; ++j) {
-            const float2 cs = tab[i0 + j];
+            const float2 cs = cs8[j];
             o[j] = lo ? rope_rot_lo(v[j], w[j], cs) : rope_rot_hi(w[j], v[j], cs);
         }
     }
@@ -135,7 +156,8 @@ hipError_t launch_rotation(RopeArgs a, int64_t numel, hipStream_t stream) {
     a.ngroups = numel / VEC;
     const int64_t blocks = (a.ngroups + 255) / 256;
     if (blocks > 0x7fffffffLL) return hipErrorInvalidConfiguration;
-    hipLaunchKernelGGL((rope_kernel<T, VEC>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
+    if (a.table) hipLaunchKernelGGL((rope_kernel<T, VEC, false>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
+    else hipLaunchKernelGGL((rope_kernel<T, VEC, true>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
     return hipGetLastError();
 }
 
@@ -166,9 +188,11 @@ hipError_t gt_launch_rope_table(const int32_t *pos, const int32_t *base, int64_t
     return hipGetLastError();
 }
 
+bool gt_rope_inline(int64_t numel, int64_t D) { return D <= kRopeInlineMaxDim && numel / 8 <= kRopeInlineThreads; }
+
 hipError_t gt_launch_rope(const void *x, int dtype, const int64_t *strides, void *y, const void *table,
                           int64_t table_b_stride, int64_t B, int64_t H, int64_t S, int64_t D, int n_dims, int mode,
-                          hipStream_t stream) {
+                          hipStream_t stream, const gt_rope_angles *angles) {
     const int64_t numel = B * H * S * D;
     if (numel <= 0) return hipSuccess;
     RopeArgs a{};
@@ -179,6 +203,14 @@ hipError_t gt_launch_rope(const void *x, int dtype, const int64_t *strides, void
     a.sd = strides[3];
     a.y = y;
     a.table = (const float2 *)table;
+    if (angles) {
+        a.pos = angles->pos;
+        a.theta_scale = angles->theta_scale;
+        a.freq_scale = angles->freq_scale;
+        a.sin_sign = angles->backward ? -1.0f : 1.0f;
+    } else if (!table) {
+        return hipErrorInvalidValue;
+    }
     a.tb = table_b_stride;
     a.H = H;
     a.S = S;

@@ -111,11 +111,17 @@ gt_tensor *rope_run(const gt_tensor *x, const gt_tensor *pos, const RopeLayout &
     }
     gt_tensor *out = ps ? gt_new_tensor(x->ndim, x->shape, x->dtype, GT_DEV_CUDA, dev) : nullptr;
     gt_scratch table;
-    bool ok = out && gt_scratch_alloc(table, (size_t)L.S * (size_t)(n_dims / 2) * 2 * sizeof(float), dev);
-    if (ok) {
-        const float theta_scale = gt_rope_theta_scale(freq_base, n_dims);
-        const int64_t strides[4] = {l.sb, l.sh, l.ss, l.sd};
-        ok = gt_hip_check(gt_launch_rope_table((const int32_t *)gt_data(ps), nullptr, 1, L.S, n_dims, theta_scale,
+    const float theta_scale = gt_rope_theta_scale(freq_base, n_dims);
+    const int64_t strides[4] = {l.sb, l.sh, l.ss, l.sd};
+    bool ok = out != nullptr;
+    if (ok && gt_rope_inline(x->numel, L.D)) {
+        const gt_rope_angles angles{(const int32_t *)gt_data(ps), theta_scale, freq_scale, backward ? 1 : 0};
+        ok = gt_hip_check(gt_launch_rope(gt_data(xs), x->dtype, strides, gt_data(out), nullptr, 0, L.B, L.H, L.S, L.D,
+                                         n_dims, mode, gt_stream(), &angles),
+                          "rope kernel");
+    } else if (ok) {
+        ok = gt_scratch_alloc(table, (size_t)L.S * (size_t)(n_dims / 2) * 2 * sizeof(float), dev) &&
+             gt_hip_check(gt_launch_rope_table((const int32_t *)gt_data(ps), nullptr, 1, L.S, n_dims, theta_scale,
                                                freq_scale, backward ? 1 : 0, table.ptr(), gt_stream()),
                           "rope table kernel") &&
              gt_hip_check(gt_launch_rope(gt_data(xs), x->dtype, strides, gt_data(out), table.ptr(), 0, L.B, L.H, L.S,
