@@ -249,6 +249,27 @@ def _configure(lib: ctypes.CDLL) -> ctypes.CDLL:
 lib = _configure(_load_native())
 
 
+def _load_bridge():
+    """The CPython module that lends tensors to the library (built with it, and checked like it)."""
+    import torch  # noqa: F401  (its libraries first: the module links to them by name)
+
+    from ._srchash import bridge_hash
+
+    try:
+        from . import _gt_bridge
+    except ImportError as e:
+        raise ImportError(f"{_PKG_DIR / '_gt_bridge.so'} is not built or does not load ({e}); build it with "
+                          "`python gguf_train_amd/_build.py`") from e
+    want = bridge_hash()
+    if want is not None and _gt_bridge.SOURCE_HASH != want:
+        raise ImportError(f"{_gt_bridge.__file__} was built from other sources; rebuild it with "
+                          "`python gguf_train_amd/_build.py`")
+    return _gt_bridge
+
+
+bridge = _load_bridge()
+
+
 def last_launch() -> str:
     """The kernels this thread's last attention call launched (gt_last_launch)."""
     msg = lib.gt_last_launch()

@@ -3,7 +3,7 @@
 Inputs are lent to the library as borrowed handles (gt_tensor_from_device_ptr for HIP
 memory, gt_tensor_from_external for host memory); results come back as library-owned
 handles and are adopted by PyTorch through DLPack (gt_tensor_to_dlpack), so the memory the
-kernels wrote is the memory the caller reads.  Every native call is made on the caller's
+kernels wrote is the memory the caller reads.  Both steps run in the native module _gt_bridge.  Every native call is made on the caller's
 current PyTorch stream (gt_set_stream), which keeps the library ordered with PyTorch work.
 
 PyTorch is plumbing here: device memory and streams.  No attention math happens in PyTorch.
@@ -35,10 +35,7 @@ GT_TO_TORCH = {v: k for k, v in TORCH_TO_GT.items()}
 
 _tokens = itertools.count(1)
 
-_PyCapsule_New = ctypes.pythonapi.PyCapsule_New
-_PyCapsule_New.restype = ctypes.py_object
-_PyCapsule_New.argtypes = [ctypes.c_void_p, ctypes.c_char_p, ctypes.c_void_p]
-_DLTENSOR = b"dltensor"
+Handle = _C.bridge.Handle  # owns one gt_tensor* (`ptr`), freed with it; `keep` pins borrowed memory
 
 
 @dataclass
@@ -66,98 +63,57 @@ class QuantizedTensor:
         return n
 
 
-class Handle:
-    """Owns one gt_tensor* and frees it when dropped; `keep` pins borrowed memory."""
-
-    __slots__ = ("ptr", "keep")
-
-    def __init__(self, ptr: int, keep=None):
-        self.ptr = ptr
-        self.keep = keep
-
-    def release(self) -> int:
-        p, self.ptr = self.ptr, 0
-        return p
-
-    def __del__(self, _free=_C.lib.gt_tensor_free):
-        if self.ptr:
-            _free(self.ptr)
-            self.ptr = 0
-
-
 def _i64(vals) -> ctypes.Array:
     vals = [int(v) for v in vals]
     return (ctypes.c_int64 * max(len(vals), 1))(*vals)
 
 
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def bind_stream(device: torch.device) -> None:
     """Makes the library enqueue on PyTorch's current stream of `device`."""
-    if device.type == "cuda":
-        _C.lib.gt_set_stream(ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream))
+    if device.type != "cuda":
+        _C.bridge.set_stream(0)
+    elif _raw_stream is not None and device.index is not None and torch.cuda.is_initialized():
+        _C.bridge.set_stream(_raw_stream(device.index))
     else:
-        _C.lib.gt_set_stream(None)
-
-
-_released_buf = (ctypes.c_uint64 * 1024)()
-
-
-def _drain_released() -> None:
-    """Borrowed memory stays pinned by `Handle.keep`, so the release tokens the library queues
-    carry no information here; drop them so the queue does not grow."""
-    while _C.lib.gt_external_released(_released_buf, 1024) == 1024:
-        pass
+        _C.bridge.set_stream(torch.cuda.current_stream(device).cuda_stream)
 
 
 def borrow(t) -> Handle:
-    """A handle on the memory of a PyTorch tensor (or QuantizedTensor), without a copy."""
-    if next(_tokens) % 512 == 0:
-        _drain_released()
-    if isinstance(t, QuantizedTensor):
-        d = t.data
-        if not d.is_cuda:
-            nb = d.numel()
-            ptr = _C.lib.gt_tensor_from_data(len(t.shape), _i64(t.shape), _C.GT_Q8_0, _C.GT_DEV_CPU, 0,
-                                             ctypes.c_void_p(d.contiguous().data_ptr()), nb)
-            return Handle(_C.check_ptr(ptr, "borrow"))
-        if not d.is_contiguous() or d.dtype != torch.uint8:
-            raise ValueError("QuantizedTensor.data must be a contiguous uint8 tensor")
-        strides = []
-        acc = 1
-        for s in reversed(t.shape):
-            strides.append(acc)
-            acc *= int(s)
-        strides.reverse()
-        ptr = _C.lib.gt_tensor_from_device_ptr(len(t.shape), _i64(t.shape), _i64(strides), _C.GT_Q8_0,
-                                               d.device.index or 0, ctypes.c_void_p(d.data_ptr()), next(_tokens))
-        return Handle(_C.check_ptr(ptr, "borrow"), keep=d)
-    if t.dtype not in TORCH_TO_GT:
-        raise TypeError(f"dtype {t.dtype} is not supported by libgt_attn")
-    code = TORCH_TO_GT[t.dtype]
-    if t.numel() == 0:
-        # nothing to lend: an empty library tensor of the same shape and device
-        dev_type = _C.GT_DEV_CUDA if t.is_cuda else _C.GT_DEV_CPU
-        ptr = _C.lib.gt_tensor_empty(t.ndim, _i64(t.shape), code, dev_type, (t.device.index or 0) if t.is_cuda else 0)
+    """A Handle (its `ptr` a gt_tensor*) on the memory of a PyTorch tensor or QuantizedTensor, without a
+    copy; it frees the gt_tensor when dropped and pins the memory until then."""
+    if not isinstance(t, QuantizedTensor):
+        return _C.bridge.borrow(t)
+    d = t.data
+    h = _C.bridge.borrow_q8(d, t.shape) if type(t.shape) is tuple and t.gt_dtype == _C.GT_Q8_0 else None
+    if h is not None:
+        return h
+    if not d.is_cuda:
+        nb = d.numel()
+        ptr = _C.lib.gt_tensor_from_data(len(t.shape), _i64(t.shape), _C.GT_Q8_0, _C.GT_DEV_CPU, 0,
+                                         ctypes.c_void_p(d.contiguous().data_ptr()), nb)
         return Handle(_C.check_ptr(ptr, "borrow"))
-    shape, strides = _i64(t.shape), _i64(t.stride())
-    if t.is_cuda:
-        ptr = _C.lib.gt_tensor_from_device_ptr(t.ndim, shape, strides, code, t.device.index or 0,
-                                               ctypes.c_void_p(t.data_ptr()), next(_tokens))
-    else:
-        ptr = _C.lib.gt_tensor_from_external(t.ndim, shape, strides, code, ctypes.c_void_p(t.data_ptr()),
-                                             next(_tokens))
-    return Handle(_C.check_ptr(ptr, "borrow"), keep=t)
+    if not d.is_contiguous() or d.dtype != torch.uint8:
+        raise ValueError("QuantizedTensor.data must be a contiguous uint8 tensor")
+    strides = []
+    acc = 1
+    for s in reversed(t.shape):
+        strides.append(acc)
+        acc *= int(s)
+    strides.reverse()
+    ptr = _C.lib.gt_tensor_from_device_ptr(len(t.shape), _i64(t.shape), _i64(strides), _C.GT_Q8_0,
+                                           d.device.index or 0, ctypes.c_void_p(d.data_ptr()), next(_tokens))
+    return Handle(_C.check_ptr(ptr, "borrow"), keep=d)
 
 
 def adopt(ptr: int, ctx: str = "") -> torch.Tensor:
     """Turns a library-owned result handle into a PyTorch tensor (zero-copy, via DLPack)."""
-    _C.check_ptr(ptr, ctx)
-    try:
-        dl = _C.lib.gt_tensor_to_dlpack(ptr)
-        _C.check_ptr(dl, ctx)
-    finally:
-        _C.lib.gt_tensor_free(ptr)
-    capsule = _PyCapsule_New(dl, _DLTENSOR, None)
-    return torch.utils.dlpack.from_dlpack(capsule)
+    t = _C.bridge.adopt(_C.check_ptr(ptr, ctx))
+    if t is None:
+        _C.check_ptr(0, ctx)
+    return t
 
 
 def adopt_quantized(ptr: int, shape, ctx: str = "") -> QuantizedTensor:

@@ -1,4 +1,5 @@
-"""In-tree build of libgt_attn.so (hipcc, gfx950).
+"""In-tree build of libgt_attn.so (hipcc, gfx950) and of _gt_bridge.so, the CPython module that lends
+PyTorch tensors to it (g++ against PyTorch's headers).
 
     python gguf_train_amd/_build.py            (a script: the package needs the library)
 
@@ -20,6 +21,8 @@ PKG_DIR = Path(__file__).resolve().parent
 CSRC = PKG_DIR / "csrc"
 OBJ_DIR = PKG_DIR / "_build"
 LIB_PATH = PKG_DIR / "libgt_attn.so"
+BRIDGE_SRC = PKG_DIR / "torch_bridge.cpp"
+BRIDGE_PATH = PKG_DIR / "_gt_bridge.so"
 ARCH = "gfx950"
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -40,14 +43,18 @@ def _sources() -> list[Path]:
     return sorted(list(CSRC.glob("*.hip")) + list(CSRC.glob("*.cpp")))
 
 
-def _source_hash() -> str:
+def _srchash():
     # loaded by path: importing the package would load the library being built
     import importlib.util
 
     spec = importlib.util.spec_from_file_location("_gt_srchash", PKG_DIR / "_srchash.py")
     mod = importlib.util.module_from_spec(spec)
     spec.loader.exec_module(mod)
-    return mod.source_hash(PKG_DIR)
+    return mod
+
+
+def _source_hash() -> str:
+    return _srchash().source_hash(PKG_DIR)
 
 
 def _generate() -> None:
@@ -87,7 +94,32 @@ def build_library(jobs: int | None = None) -> Path:
     if proc.returncode != 0:
         raise RuntimeError(f"link failed:\n{' '.join(cmd)}\n{proc.stdout}\n{proc.stderr}")
     os.replace(tmp, LIB_PATH)
+    build_bridge()
     return LIB_PATH
+
+
+def build_bridge() -> Path:
+    """_gt_bridge.so, linked to the library beside it."""
+    import sysconfig
+    from importlib.util import find_spec
+
+    torch_dir = Path(find_spec("torch").origin).resolve().parent
+    inc, lib = torch_dir / "include", torch_dir / "lib"
+    obj, tmp = OBJ_DIR / "torch_bridge.cpp.o", BRIDGE_PATH.with_suffix(".so.tmp")
+    digest = _srchash().bridge_hash(PKG_DIR)
+    OBJ_DIR.mkdir(exist_ok=True)
+    for cmd in (
+        ["g++", "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-Wall", f'-DGT_BRIDGE_HASH="{digest}"',
+         f"-I{sysconfig.get_paths()['include']}", f"-isystem{inc}", f"-isystem{inc}/torch/csrc/api/include", "-c",
+         str(BRIDGE_SRC), "-o", str(obj)],
+        ["g++", "-shared", "-o", str(tmp), str(obj), f"-L{PKG_DIR}", "-l:libgt_attn.so", f"-L{lib}", "-ltorch_python",
+         "-ltorch_cpu", "-lc10", "-Wl,-rpath,$ORIGIN"],
+    ):
+        proc = subprocess.run(cmd, capture_output=True, text=True)
+        if proc.returncode != 0:
+            raise RuntimeError(f"{cmd[0]} failed:\n{' '.join(cmd)}\n{proc.stdout}\n{proc.stderr}")
+    os.replace(tmp, BRIDGE_PATH)
+    return BRIDGE_PATH
 
 
 def main(argv: list[str]) -> int:

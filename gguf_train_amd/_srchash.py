@@ -32,3 +32,11 @@ def source_hash(pkg_dir: Path = PKG_DIR) -> str | None:
         h.update(p.read_bytes())
         h.update(b"\0")
     return h.hexdigest()
+
+
+def bridge_hash(pkg_dir: Path = PKG_DIR) -> str | None:
+    """Hex SHA-256 of the PyTorch bridge's source and the ABI it calls, or None when not present."""
+    files = [pkg_dir / "torch_bridge.cpp", pkg_dir.parent / "include" / "gt_attn.h"]
+    if not all(p.is_file() for p in files):
+        return None
+    return hashlib.sha256(b"\0".join(p.read_bytes() for p in files)).hexdigest()

@@ -30,6 +30,8 @@ from .. import _ops
 def _autocast_lower(*ts):
     """Casts floating-point operands to the active autocast dtype (the reference's
     _AUTOCAST_LOWER policy); returns them unchanged outside autocast."""
+    if not (torch.is_autocast_enabled("cuda") or torch.is_autocast_enabled("cpu")):
+        return ts
     out = []
     for t in ts:
         if isinstance(t, torch.Tensor) and t.is_floating_point():
@@ -63,19 +65,23 @@ def scaled_dot_product_attention(
                 )
             if attn_mask.ndim != 4:
                 attn_mask = attn_mask.reshape((1,) * (4 - attn_mask.ndim) + tuple(attn_mask.shape))
-    quantized = isinstance(key, QuantizedTensor) or isinstance(value, QuantizedTensor)
-    with torch.autocast(query.device.type, enabled=False):
-        if quantized:
-            if dropout_p != 0.0:
-                raise RuntimeError("scaled_dot_product_attention: dropout is not supported with q8_0 key/value")
-            return _ops.flash_attention(query, key, value, attn_mask, sc, is_causal)
-        if dropout_p == 0.0:
-            return FlashAttentionFn.apply(query, key, value, attn_mask, sc, is_causal)
-        # dropout (the reference composes it, gguf_train/nn/functional.py:750-767): fused forward
-        # and backward drawing the decisions from a seed of torch's generator
-        out, _ = FlashAttentionDropoutFn.apply(query, key, value, attn_mask, sc, is_causal, float(dropout_p),
-                                               draw_dropout_seed())
-        return out
+    if torch.is_autocast_enabled(query.device.type):  # (entering the context costs a few us)
+        with torch.autocast(query.device.type, enabled=False):
+            return _attend(query, key, value, attn_mask, float(dropout_p), is_causal, sc)
+    return _attend(query, key, value, attn_mask, float(dropout_p), is_causal, sc)
+
+
+def _attend(query, key, value, attn_mask, dropout_p: float, is_causal: bool, sc: float):
+    if isinstance(key, QuantizedTensor) or isinstance(value, QuantizedTensor):
+        if dropout_p != 0.0:
+            raise RuntimeError("scaled_dot_product_attention: dropout is not supported with q8_0 key/value")
+        return _ops.flash_attention(query, key, value, attn_mask, sc, is_causal)
+    if dropout_p == 0.0:
+        return FlashAttentionFn.apply(query, key, value, attn_mask, sc, is_causal)
+    # dropout (the reference composes it, gguf_train/nn/functional.py:750-767): fused forward
+    # and backward drawing the decisions from a seed of torch's generator
+    out, _ = FlashAttentionDropoutFn.apply(query, key, value, attn_mask, sc, is_causal, dropout_p, draw_dropout_seed())
+    return out
 
 
 def rope(input, positions, n_dims: int | None = None, mode: int = 0, n_ctx_orig: int = 0, freq_base: float = 10000.0,
