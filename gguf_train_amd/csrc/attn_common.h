@@ -179,10 +179,15 @@ int attn_decode_splits(const AttnFwdArgs &f, int cd);
 int attn_decode_max_tile(int cd);  // query heads per workgroup at most (decode_units' max_tile)
 hipError_t launch_attn_decode(const DecodeArgs &a, int cd, hipStream_t s);
 
+// Head sizes of the half-precision prefill and backward kernels (float32: 64 and 128).  Single query rows
+// of 80 and 96 keep the generic kernels.
+inline bool attn_half_head(int64_t D, int64_t L) { return D == 64 || D == 128 || ((D == 80 || D == 96) && L > 1); }
+
 bool attn_prefill_supported(const AttnFwdArgs &f, int cd);
 // (launch_attn_prefill runs the software-pipelined fp16 head-size-128 kernel where
 // attn_prefill_asm_supported holds, the HIP prefill kernel otherwise)
 hipError_t launch_attn_prefill(const AttnFwdArgs &a, int cd, hipStream_t s);
+hipError_t launch_prefill_heads(const AttnFwdArgs &a, int cd, int nq, int order, int64_t grid, hipStream_t s);  // D = 80, 96
 int attn_prefill_key_tile(const AttnFwdArgs &f);  // keys per tile of the half-precision kernel
 // Fills t.cls and t.bits from a mask of `batches` (L, S) planes; kind 0 bool bytes, 1 float16, 2
 // bfloat16, 3 float32; copy: float32 values of the half-precision kinds' kMaskTileValues tiles.
@@ -207,3 +212,4 @@ hipError_t launch_dropout_mask(const GtDropout &d, bool keep_all, int64_t rows, 
 bool attn_bwd_mfma_supported(const AttnBwdArgs &a, int cd);
 bool attn_bwd_f32_split(const AttnBwdArgs &a);  // float32: the small-grid backward kernels
 hipError_t launch_attn_bwd_mfma(const AttnBwdArgs &a, int cd, hipStream_t s);
+hipError_t launch_attn_bwd_heads(const AttnBwdArgs &a, int cd, hipStream_t s);  // D = 80, 96 (half precision)

@@ -391,22 +391,35 @@ void apply_dropout(AttnFwdArgs &a, const Dropout *drop) {
 }
 
 // ---- head padding ----------------------------------------------------------------------------
-// The MFMA kernels take head sizes 64 and 128.  Attention with another head size up to 128 and
-// more than one query row runs on them with q, k, v (and in the backward dO and the output)
-// zero-padded to 64 or 128 dims: the zero dims add nothing to Q.K^T (the scale stays that of the
-// real head size), padded V columns give output columns that are dropped, and the padded columns
-// of dQ, dK, dV are zero and dropped.  Single-query rows keep their kernels (padding would copy
-// the whole K/V).  Float32 pads only calls its MFMA kernels take (16 query rows or more, no KV
+// The MFMA kernels take head sizes 64 and 128, the half-precision ones 80 and 96 as well.  Attention with
+// another head size up to 128 and more than one query row runs on them with q, k, v (and in the backward
+// dO and the output) zero-padded to the next of these: the zero dims add nothing to Q.K^T (the scale
+// stays that of the real head size), padded V columns give output columns that are dropped, and the
+// padded columns of dQ, dK, dV are zero and dropped.  Single-query rows keep their kernels (padding would
+// copy the whole K/V).  Float32 pads only calls its MFMA kernels take (16 query rows or more, no KV
 // cache lengths: f32_pads; the backward also 32 dQ workgroups), the rest keep the generic kernels
 // unpadded.
-int64_t mfma_head(int64_t d) { return d <= 0 ? 0 : d <= 64 ? 64 : d <= 128 ? 128 : 0; }
+// 80 and 96 have kernels of their own because padding them to 128 costs a pass over every operand and
+// result, and a third to a half more matrix work: training step of fp16 B4 H16 L1000 D80 causal, 263 us
+// padded to 128 (92 us of it copies), 133 us read in place.
+int64_t mfma_head(int cd, int64_t d) {
+    if (d <= 0 || d > 128) return 0;
+    if (d <= 64) return 64;
+    return cd == GT_F32 || d > 96 ? 128 : d <= 80 ? 80 : 96;
+}
 
 int64_t padded_head(int cd, int64_t L, int64_t D, int64_t Dv) {
     if ((cd != GT_F16 && cd != GT_BF16 && cd != GT_F32) || L <= 1) return 0;
     if (cd == GT_F32 && L < 16) return 0;
-    if (D == Dv && (D == 64 || D == 128)) return 0;
-    if (!mfma_head(D) || !mfma_head(Dv)) return 0;
-    return std::max(mfma_head(D), mfma_head(Dv));
+    const int64_t p = std::max(mfma_head(cd, D), mfma_head(cd, Dv));
+    if (!mfma_head(cd, D) || !mfma_head(cd, Dv) || (D == p && Dv == p)) return 0;
+    return p;
+}
+
+// Calls of a head size between 64 and 128 that need no padding but whose rows the kernels cannot read in
+// place (starts off 16 bytes, strides off 8 elements) are copied dense: pad_heads to their own size.
+bool copies_rows(int cd, int64_t L, int64_t D, int64_t Dv) {
+    return (cd == GT_F16 || cd == GT_BF16) && L > 1 && D == Dv && D > 64 && D < 128 && mfma_head(cd, D) == D;
 }
 
 // Float32 calls whose padded form the float32 MFMA kernels take (masks staged, dropout applied).
@@ -514,7 +527,9 @@ int attention_forward(const char *who, const gt_tensor *q, const gt_tensor *k, c
             apply_dropout(a, drop);
             // heads padded to the MFMA kernels' sizes (output and float32 output unpadded after)
             const gt_tensor *po = nullptr, *po32 = nullptr;
-            const int64_t Dp = qrope || a.out_dtype != cd || (cd == GT_F32 && !f32_pads(a)) ? 0 : padded_head(cd, L, D, Dv);
+            const bool pads = !qrope && a.out_dtype == cd && (cd != GT_F32 || f32_pads(a));
+            int64_t Dp = pads ? padded_head(cd, L, D, Dv) : 0;
+            if (pads && !Dp && copies_rows(cd, L, D, Dv) && !attn_prefill_supported(a, cd)) Dp = D;
             if (Dp) {
                 const gt_tensor *qp = pad_heads(qs, Dp, dev, tmp), *kp = pad_heads(ks, Dp, dev, tmp);
                 const gt_tensor *vp = pad_heads(vs, Dp, dev, tmp);
@@ -714,7 +729,7 @@ int attention_backward(const char *who, const gt_tensor *grad_out, const gt_tens
     // it is the training forward's copy bit for bit).
     const gt_tensor *lse_s = nullptr, *out_s = nullptr;
     int64_t Dp = padded_head(cd, L, D, Dv);  // heads padded for the MFMA kernels (0: none)
-    const bool mfma_shape = ((cd == GT_F16 || cd == GT_BF16) && D == Dv && (D == 64 || D == 128)) || Dp != 0;
+    const bool mfma_shape = ((cd == GT_F16 || cd == GT_BF16) && D == Dv && attn_half_head(D, L)) || Dp != 0;
     if (!lse || !out || (mfma_shape && out->dtype != GT_F32)) {
         gt_tensor *o2 = nullptr, *l2 = nullptr, *o32 = nullptr;
         if (attention_forward(who, q, k, v, mask, scale, is_causal, &o2, &l2, mfma_shape ? &o32 : nullptr, nullptr,
@@ -764,6 +779,7 @@ int attention_backward(const char *who, const gt_tensor *grad_out, const gt_tens
         a.f.o = const_cast<void *>(gt_data(out_s));
         a.o_f32 = od == GT_F32 && cd != GT_F32;
         apply_dropout(a.f, drop);
+        if (!Dp && copies_rows(cd, L, D, Dv) && !attn_bwd_mfma_supported(a, cd)) Dp = D;
         a.g_half = half_ok && (Dp || attn_bwd_mfma_supported(a, cd)) ? 1 : 0;
         const int kd = a.g_half ? cd : gd;
         gq = gt_new_tensor(4, qsh, kd, GT_DEV_CUDA, dev);
@@ -1641,7 +1657,14 @@ extern "C" gt_tensor *gt_kv_cache_attention(gt_kv_cache *c, const gt_tensor *q, 
         ok = qs && ks && vs;
         // heads padded to the MFMA kernels' sizes (the cache's first maxlen rows are copied)
         const gt_tensor *po = nullptr;
-        const int64_t Dp = ok && q->dtype == cd ? padded_head(cd, L, D, D) : 0;
+        int64_t Dp = ok && q->dtype == cd ? padded_head(cd, L, D, D) : 0;
+        if (ok && q->dtype == cd && !Dp && copies_rows(cd, L, D, D)) {
+            AttnFwdArgs probe{};
+            fill_qkv(probe, qs, ks, vs);
+            probe.scale = scale;
+            probe.out_dtype = cd;
+            if (!attn_prefill_supported(probe, cd)) Dp = D;
+        }
         if (Dp) {
             const gt_tensor *qp = pad_heads(qs, Dp, dev, tmp), *kp = pad_heads(ks, Dp, dev, tmp);
             const gt_tensor *vp = pad_heads(vs, Dp, dev, tmp);
