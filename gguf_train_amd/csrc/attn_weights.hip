@@ -238,7 +238,10 @@ __global__ __launch_bounds__(64 * WQ) void attn_weights_vec_kernel(AttnFwdArgs f
 // k-steps at a time from one 16-byte load of key row lrow.  The wavefront's 32 x 64 tile goes
 // through LDS (16-byte writes, rows padded by 16 bytes) and out as 16-byte pieces when S % 4 == 0
 // and the output is 16-byte aligned (VEC), else as 4-byte stores of 64 consecutive keys.
-template <int D, bool CAUSAL, int MASK, bool AVG, bool VEC>
+// HS (averaged weights of small grids): the wavefronts of a workgroup share 32 query rows and take the
+// heads w, w + 4, ..; their tiles are added in LDS.  A wavefront's walk over the heads is a chain of
+// loads, products and exponentials, so it bounds a grid that leaves SIMDs idle.
+template <int D, bool CAUSAL, int MASK, bool AVG, bool VEC, bool HS>
 __global__ __launch_bounds__(64 * WQ) void attn_weights_f32_kernel(AttnFwdArgs f, void *wout, int64_t nrb) {
     constexpr int DH = D / 2;
     constexpr int RP = 64 + 4;  // LDS row pitch (floats): 64 keys and 16 bytes of padding
@@ -248,7 +251,7 @@ __global__ __launch_bounds__(64 * WQ) void attn_weights_f32_kernel(AttnFwdArgs f
     const int64_t rb = blockIdx.x % nrb, g = blockIdx.x / nrb;
     const int64_t b = AVG ? g : g / f.H;
     const int L = (int)f.L, S = (int)f.S;
-    const int q0 = (int)rb * 32 * WQ + 32 * w;  // first query row of this wavefront
+    const int q0 = HS ? (int)rb * 32 : (int)rb * 32 * WQ + 32 * w;  // first query row of this wavefront
     const int q = q0 + lrow;                    // this lane's query row
     const int qc = min(q, L - 1);
     const float c = f.scale * kLog2e;
@@ -279,7 +282,7 @@ __global__ __launch_bounds__(64 * WQ) void attn_weights_f32_kernel(AttnFwdArgs f
         for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
             for (int i = 0; i < 16; ++i) acc[kb][i] = 0.0f;
-        for (int hh = 0; hh < nh; ++hh) {
+        for (int hh = HS ? w : 0; hh < nh; hh += HS ? WQ : 1) {
             const int64_t h = AVG ? hh : g % f.H;
             const int64_t hk = h / (f.H / f.Hkv);
             float ls = ls1;
@@ -293,6 +296,16 @@ __global__ __launch_bounds__(64 * WQ) void attn_weights_f32_kernel(AttnFwdArgs f
                 }
                 ls = ((const float *)f.lse)[(b * f.H + h) * f.L + qc] * kLog2e;
             }
+            f32x4 kpre[HS ? 2 : 1][DH / 4];  // HS: both key blocks' K in flight at once
+            if constexpr (HS) {
+#pragma unroll
+                for (int kb = 0; kb < 2; ++kb) {
+                    const float *kr = (const float *)f.k + b * f.k_sb + hk * f.k_sh +
+                                      (int64_t)min(k0 + 32 * kb + lrow, S - 1) * f.k_ss + DH * half;
+#pragma unroll
+                    for (int u = 0; u < DH / 4; ++u) kpre[kb][u] = *(const f32x4 *)(kr + 4 * u);
+                }
+            }
 #pragma unroll
             for (int kb = 0; kb < 2; ++kb) {
                 const int kb0 = k0 + 32 * kb;
@@ -305,7 +318,7 @@ __global__ __launch_bounds__(64 * WQ) void attn_weights_f32_kernel(AttnFwdArgs f
                 for (int i = 0; i < 16; ++i) sc[i] = 0.0f;
 #pragma unroll
                 for (int u = 0; u < DH / 4; ++u) {
-                    const f32x4 kv = *(const f32x4 *)(kr + 4 * u);
+                    const f32x4 kv = HS ? kpre[kb][u] : *(const f32x4 *)(kr + 4 * u);
 #pragma unroll
                     for (int e = 0; e < 4; ++e) sc = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[e], qf[4 * u + e], sc, 0, 0, 0);
                 }
@@ -329,7 +342,8 @@ __global__ __launch_bounds__(64 * WQ) void attn_weights_f32_kernel(AttnFwdArgs f
             }
         }
         // the tile into LDS as rows (query) x keys, four keys per 16-byte write
-        __builtin_amdgcn_wave_barrier();  // the previous tile's reads are done
+        if constexpr (HS) __syncthreads();  // the previous tile's reads are done
+        else __builtin_amdgcn_wave_barrier();
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
@@ -337,21 +351,40 @@ __global__ __launch_bounds__(64 * WQ) void attn_weights_f32_kernel(AttnFwdArgs f
                 const f32x4 v4 = {acc[kb][4 * gq], acc[kb][4 * gq + 1], acc[kb][4 * gq + 2], acc[kb][4 * gq + 3]};
                 *(f32x4 *)&tw[lrow * RP + 32 * kb + 8 * gq + 4 * half] = v4;
             }
-        __builtin_amdgcn_wave_barrier();
-        if constexpr (VEC) {
-            // piece u * 64 + lane: row (u * 64 + lane) / 16, keys 4 * (lane % 16) .. +3
+        if constexpr (HS) __syncthreads();
+        else __builtin_amdgcn_wave_barrier();
+        // the value(s) at `at` of the 32 x 64 tile: this wavefront's own, or all four's sum
+        auto out4 = [&](int at) {
+            if constexpr (!HS) return *(const f32x4 *)&tw[at];
+            f32x4 x = *(const f32x4 *)&tile[0][at];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const int pc = u * 64 + lane, row = pc >> 4, key0 = k0 + 4 * (pc & 15);
-                const f32x4 piece = *(const f32x4 *)&tw[row * RP + 4 * (pc & 15)];
+            for (int o = 1; o < WQ; ++o) x += *(const f32x4 *)&tile[o][at];
+            return x;
+        };
+        auto out1 = [&](int at) {
+            if constexpr (!HS) return tw[at];
+            float x = tile[0][at];
+#pragma unroll
+            for (int o = 1; o < WQ; ++o) x += tile[o][at];
+            return x;
+        };
+        // the rows this wavefront writes
+        constexpr int RW = HS ? 32 / WQ : 32;
+        const int r0 = HS ? RW * w : 0;
+        if constexpr (VEC) {
+            // piece u * 64 + lane: row r0 + (u * 64 + lane) / 16, keys 4 * (lane % 16) .. +3
+#pragma unroll
+            for (int u = 0; u < RW / 4; ++u) {
+                const int pc = u * 64 + lane, row = r0 + (pc >> 4), key0 = k0 + 4 * (pc & 15);
+                const f32x4 piece = out4(row * RP + 4 * (pc & 15));
                 if (q0 + row < L && key0 < S) *(f32x4 *)((float *)wout + (base + q0 + row) * f.S + key0) = piece;
             }
         } else {
             // row r: lanes write its 64 keys
 #pragma unroll 4
-            for (int r = 0; r < 32; ++r) {
+            for (int r = r0; r < r0 + RW; ++r) {
                 const int key = k0 + lane;
-                if (q0 + r < L && key < S) ((float *)wout)[(base + q0 + r) * f.S + key] = tw[r * RP + lane];
+                if (q0 + r < L && key < S) ((float *)wout)[(base + q0 + r) * f.S + key] = out1(r * RP + lane);
             }
         }
     }
@@ -421,6 +454,13 @@ unsigned key_splits(int64_t grid, int64_t nkt, bool avg) {
     return (unsigned)std::max<int64_t>(1, std::min<int64_t>(nkt, (1024 + grid - 1) / grid));
 }
 
+// Averaged float32 weights whose heads are split over a workgroup's wavefronts (`grid`: workgroups of 128
+// query rows, nkt: 64-key tiles): while the unsplit grid has less than one workgroup for each of the 256
+// CUs.  From there on the SIMDs are busy either way, and Q and K are loaded by four times the workgroups
+// (D64 H8, key padding, unsplit against split: B8 L=S=256, 64 workgroups, 56.9 against 19.3 us; B4 L=S=512,
+// 128, 57.9 against 34.8; B8 L=S=512, 256, 61.6 against 66.8; B16, 512, 119.6 against 130.5).
+bool f32_heads_split(int64_t grid, int64_t nkt, int64_t H) { return H >= WQ && grid * nkt < 256; }
+
 template <typename T, int D, bool AVG>
 hipError_t launch_mfma(const AttnFwdArgs &f, void *w, hipStream_t st) {
     const int64_t nrb = (f.L + 32 * WQ - 1) / (32 * WQ);
@@ -450,16 +490,22 @@ hipError_t launch_mfma(const AttnFwdArgs &f, void *w, hipStream_t st) {
 
 template <int D, bool AVG>
 hipError_t launch_f32(const AttnFwdArgs &f, void *w, hipStream_t st) {
-    const int64_t nrb = (f.L + 32 * WQ - 1) / (32 * WQ);
+    int64_t nrb = (f.L + 32 * WQ - 1) / (32 * WQ);
+    const bool hs = AVG && f32_heads_split(nrb * f.B, (f.S + 63) / 64, f.H);
+    if (hs) nrb = (f.L + 31) / 32;
     const int64_t grid = nrb * (AVG ? f.B : f.B * f.H);
     if (grid > 0x7fffffffLL) return hipErrorInvalidConfiguration;
     const int mode = !f.mask ? 0 : (f.mask_bool ? 1 : 2);
     const bool vec = f.S % 4 == 0 && (uintptr_t)w % 16 == 0;
     const unsigned ny = key_splits(grid, (f.S + 63) / 64, AVG);
-#define GT_WF(C, MK)                                                                                                    \
-    do {                                                                                                                \
-        if (vec) hipLaunchKernelGGL((attn_weights_f32_kernel<D, C, MK, AVG, true>), dim3((unsigned)grid, ny), dim3(64 * WQ), 0, st, f, w, nrb); \
-        else hipLaunchKernelGGL((attn_weights_f32_kernel<D, C, MK, AVG, false>), dim3((unsigned)grid, ny), dim3(64 * WQ), 0, st, f, w, nrb); \
+#define GT_WF_HS(C, MK, V, HS_) \
+    hipLaunchKernelGGL((attn_weights_f32_kernel<D, C, MK, AVG, V, HS_>), dim3((unsigned)grid, ny), dim3(64 * WQ), 0, st, f, w, nrb)
+#define GT_WF(C, MK)                                  \
+    do {                                              \
+        if (hs && vec) GT_WF_HS(C, MK, true, AVG);    \
+        else if (hs) GT_WF_HS(C, MK, false, AVG);     \
+        else if (vec) GT_WF_HS(C, MK, true, false);   \
+        else GT_WF_HS(C, MK, false, false);           \
     } while (0)
     if (f.causal) {
         if (mode == 0) GT_WF(true, 0);
@@ -471,6 +517,7 @@ hipError_t launch_f32(const AttnFwdArgs &f, void *w, hipStream_t st) {
         else GT_WF(false, 2);
     }
 #undef GT_WF
+#undef GT_WF_HS
     return hipGetLastError();
 }
 
