@@ -317,7 +317,10 @@ __device__ inline void load8(const void *base, int64_t e0, float *v) {
 // a Q8_0 cache quantizes with four threads per block (the block's |x| max by two lane
 // exchanges) and the operations of q8_0_quantize_lane.
 // blockIdx.y picks one of up to two tensors (keys and values), of which the first is rotated; with
-// pos_next, the first workgroup writes the lengths after the append.
+// pos_next, the first workgroup writes the lengths after the append.  A decode step's append is a chain of
+// latencies (position, angles, rows), not bandwidth: I, the type that indexes threads and rows, is int32_t
+// wherever they fit (a 64-bit division is about 100 dependent instructions), and the source rows are
+// loaded before the angles are formed (Q8_0, B4 Hkv8 T1 D128 with RoPE: 8.6 -> 6.5 us).
 struct KvAppendVec {
     const void *src[2];
     void *dst[2];
@@ -330,53 +333,63 @@ struct KvAppendVec {
     int n_dims, neox;  // n_dims 0: no rotation
     float theta_scale, freq_scale;
 };
-template <int SDT, int DDT>
+template <int SDT, int DDT, typename I>
 __global__ __launch_bounds__(256) void kv_append_vec_kernel(KvAppendVec a) {
     const void *__restrict__ src = a.src[blockIdx.y];
     void *__restrict__ dst = a.dst[blockIdx.y];
     const int32_t *__restrict__ pos = a.pos;
     const int64_t s_sb = a.st[blockIdx.y][0], s_sh = a.st[blockIdx.y][1], s_st = a.st[blockIdx.y][2];
     const int Hkv = a.Hkv, T = a.T, D = a.D, n_dims = blockIdx.y == 0 ? a.n_dims : 0, neox = a.neox;
-    const int64_t cap = a.cap, n8 = a.n8;
+    const int64_t cap = a.cap;
+    const I n8 = (I)a.n8;
     if (a.pos_next && blockIdx.x == 0 && blockIdx.y == 0)
         for (int b = threadIdx.x; b < a.B; b += 256) a.pos_next[b] = pos[b] + T;
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const I i = (I)blockIdx.x * 256 + (I)threadIdx.x;
     const bool live = i < n8;
-    const int64_t ic = live ? i : 0;
-    const int per = D / 8;
+    const I ic = live ? i : 0;
+    const int per = D / 8, half = n_dims / 2;
+    const I r = ic / per;  // source row (b, h, t)
+    const int j = (int)(ic - r * per);
+    const I bh = r / T;
+    const int t = (int)(r - bh * T);
+    const I b = bh / Hkv;
+    const int h = (int)(bh - b * Hkv);
+    const int d0 = 8 * j;
+    const bool rotated = d0 < n_dims;
+    const bool lo_chunk = d0 < half;  // NeoX: the whole chunk is on one side of half
+    const int64_t srow = b * s_sb + h * s_sh + t * s_st;
+    float v[8], w[8];
+    load8<SDT>(src, srow + d0, v);
+    if (rotated && neox) load8<SDT>(src, srow + (lo_chunk ? d0 + half : d0 - half), w);
+    const int32_t p0 = pos[b];
     __shared__ float2 s_cs[kRopeInlineEntries];
-    const int64_t r0 = (int64_t)blockIdx.x * 256 / per;  // the workgroup's first row
+    const I r0 = (I)blockIdx.x * 256 / per;  // the workgroup's first row
     if (n_dims && !a.table) {
         // the rows' angles: one set per sequence for a single token, else one per row
-        const int half = n_dims / 2;
-        const int64_t rl = min((int64_t)blockIdx.x * 256 + 255, n8 - 1) / per;
-        const int n = (int)(T == 1 ? rl / Hkv - r0 / Hkv + 1 : rl - r0 + 1) * half;
+        const I rl = min((I)blockIdx.x * 256 + 255, n8 - 1) / per;
+        const I b0 = r0 / Hkv;  // (T == 1: the first sequence)
+        const int n = (int)(T == 1 ? rl / Hkv - b0 + 1 : rl - r0 + 1) * half;
         for (int e = threadIdx.x; e < n; e += 256) {
-            const int64_t rr = T == 1 ? (r0 / Hkv + e / half) * Hkv : r0 + e / half;
-            s_cs[e] = rope_cos_sin(rope_theta(pos[rr / T / Hkv] + (int)(rr % T), e % half, a.theta_scale), a.freq_scale);
+            const int er = e / half;
+            I eb;
+            int et = 0;
+            if (T == 1) {
+                eb = b0 + er;
+            } else {
+                const I ebh = (r0 + er) / T;
+                et = (int)(r0 + er - ebh * T);
+                eb = ebh / Hkv;
+            }
+            s_cs[e] = rope_cos_sin(rope_theta(pos[eb] + et, e - er * half, a.theta_scale), a.freq_scale);
         }
         __syncthreads();
     }
-    const int j = (int)(ic % per);
-    const int64_t r = ic / per;  // source row (b, h, t)
-    const int t = (int)(r % T);
-    const int64_t bh = r / T;
-    const int h = (int)(bh % Hkv);
-    const int64_t b = bh / Hkv;
-    const int d0 = 8 * j;
-    const int64_t srow = b * s_sb + h * s_sh + (int64_t)t * s_st;
-    float v[8];
-    load8<SDT>(src, srow + d0, v);
-    if (d0 < n_dims) {
-        const int half = n_dims / 2;
-        const bool lo_chunk = d0 < half;  // NeoX: the whole chunk is on one side of half
-        float w[8];
-        if (neox) load8<SDT>(src, srow + (lo_chunk ? d0 + half : d0 - half), w);
+    if (rotated) {
         // the chunk's pairs in order: first, first + 1, ...
         const int first = neox ? (lo_chunk ? d0 : d0 - half) : d0 >> 1, np = neox ? 8 : 4;
         float2 cs8[8];
         const float2 *tab = a.table ? a.table + ((int64_t)b * T + t) * half
-                                    : s_cs + (int)(T == 1 ? bh / Hkv - r0 / Hkv : r - r0) * half;
+                                    : s_cs + (int)(T == 1 ? b - r0 / Hkv : r - r0) * half;
 #pragma unroll
         for (int e = 0; e < 8; ++e)
             if (e < np) cs8[e] = tab[first + e];
@@ -394,7 +407,7 @@ __global__ __launch_bounds__(256) void kv_append_vec_kernel(KvAppendVec a) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] = rr[e];
     }
-    const int64_t row = ((int64_t)b * Hkv + h) * cap + pos[b] + t;
+    const int64_t row = ((int64_t)b * Hkv + h) * cap + p0 + t;
     if constexpr (DDT == GT_Q8_0) {
         // the four threads of a block are lanes 4k .. 4k+3 (D / 8 is a multiple of 4), all live or
         // none (n8 is too)
@@ -661,7 +674,12 @@ hipError_t gt_launch_fill_zero(void *p, int64_t bytes, hipStream_t stream) {
 template <int SDT>
 hipError_t launch_kv_append_vec(const KvAppendVec &a, int ntensors, int ddt, hipStream_t stream) {
     const dim3 grid((unsigned)((a.n8 + 255) / 256), (unsigned)ntensors);
-#define GT_KV_APPEND_VEC(DDT) hipLaunchKernelGGL((kv_append_vec_kernel<SDT, DDT>), grid, dim3(256), 0, stream, a)
+    const bool wide = (int64_t)grid.x * 256 > 0x7fffffffLL;
+#define GT_KV_APPEND_VEC(DDT)                                                                              \
+    do {                                                                                                   \
+        if (wide) hipLaunchKernelGGL((kv_append_vec_kernel<SDT, DDT, int64_t>), grid, dim3(256), 0, stream, a); \
+        else hipLaunchKernelGGL((kv_append_vec_kernel<SDT, DDT, int32_t>), grid, dim3(256), 0, stream, a); \
+    } while (0)
     if (ddt == GT_F32) GT_KV_APPEND_VEC(GT_F32);
     else if (ddt == GT_F16) GT_KV_APPEND_VEC(GT_F16);
     else if (ddt == GT_BF16) GT_KV_APPEND_VEC(GT_BF16);

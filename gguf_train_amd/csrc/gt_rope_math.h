@@ -11,10 +11,19 @@
 #include <hip/hip_runtime.h>
 
 // Angle of pair i at position p: theta_i is the float32 chain of i products (one rounding each), as
-// ggml forms it; theta_{i+1} = theta_i * theta_scale continues it.
+// ggml forms it; theta_{i+1} = theta_i * theta_scale continues it.  The chain's length differs between
+// the lanes, so it is walked 8, 4, 2 and 1 products at a time: one product per iteration spends most of a
+// wavefront's time on the loop.
 __device__ inline float rope_theta(int32_t p, int i, float theta_scale) {
     float theta = (float)p;
-    for (int j = 0; j < i; ++j) theta *= theta_scale;
+    auto times = [&](int n) {
+#pragma unroll
+        for (int j = 0; j < n; ++j) theta *= theta_scale;
+    };
+    for (int j = i >> 3; j > 0; --j) times(8);
+    if (i & 4) times(4);
+    if (i & 2) times(2);
+    if (i & 1) times(1);
     return theta;
 }
 __device__ inline float2 rope_cos_sin(float theta, float freq_scale) {
@@ -25,7 +34,7 @@ __device__ inline float2 rope_cos_sin(float theta, float freq_scale) {
 // Threads (of a kernel that rotates up to 8 elements each) up to which a workgroup forms its rows' angles
 // itself, into LDS; more of them share a table made by a launch before, since a prompt's workgroups
 // would repeat each angle for every head.  A decode step's rows then take one launch: RoPE of fp16 B4
-// H32 D128 3.2 + 5.2 -> 5.6 us.  (Every thread forming its own 8 angles took 7.6 us: one accurate
+// H32 D128 3.2 + 5.2 -> 3.9 us.  (Every thread forming its own 8 angles took 7.6 us: one accurate
 // sincosf after the other.)
 constexpr int64_t kRopeInlineThreads = 65536;
 constexpr int kRopeInlineMaxDim = 256;  // head size up to which the angles of a workgroup's rows fit
