@@ -437,6 +437,16 @@ const gt_tensor *pad_heads(const gt_tensor *t, int64_t Dp, int dev, Temps &tmp) 
     return p;
 }
 
+// A dense copy of the 4-D tensor t in dtype cd, kept in tmp.  Rows of a device tensor of that dtype move in
+// 16-byte pieces where they allow it: the (B, L, H, D) gradient of a transposed output, float32 B8 H8 L256
+// D64, 11.8 -> 4.8 us.
+const gt_tensor *dense_rows(const gt_tensor *t, int cd, int dev, Temps &tmp) {
+    if (t->ndim == 4 && t->device_type == GT_DEV_CUDA && t->device_index == dev && t->dtype == cd && t->strides[3] == 1 &&
+        cd != GT_F64)
+        return pad_heads(t, t->shape[3], dev, tmp);
+    return tmp.keep(gt_to_device_dense(t, dev, cd));
+}
+
 // The first t->shape[3] dims of every row of the dense padded buffer `src` into the dense t.
 bool unpad_heads(const gt_tensor *src, gt_tensor *t) {
     const int64_t rows = t->shape[0] * t->shape[1] * t->shape[2];
@@ -761,7 +771,7 @@ int attention_backward(const char *who, const gt_tensor *grad_out, const gt_tens
     const gt_tensor *gos = grad_out->device_type == GT_DEV_CUDA && grad_out->device_index == dev &&
                                    grad_out->dtype == cd && gt_is_dense(grad_out)
                                ? grad_out
-                               : tmp.keep(gt_to_device_dense(grad_out, dev, cd));
+                               : dense_rows(grad_out, cd, dev, tmp);
     bool ok = delta && qs && ks && vs && gos && lse_s;
     AttnBwdArgs a{};
     if (ok) {
