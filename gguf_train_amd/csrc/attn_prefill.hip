@@ -560,7 +560,8 @@ bool attn_prefill_supported(const AttnFwdArgs &f, int cd) {
     if (f.rope_q && f.mask && (f.mask_bool || f.m_sl != 0)) return false;  // fused RoPE: no mask or key padding
     if (f.rope_q && f.dropout) return false;
     if (f.out_dtype != cd || f.D != f.Dv || !attn_half_head(f.D, f.L)) return false;
-    if (f.rope_q && f.D != 64 && f.D != 128) return false;
+    // 80 and 96: no fused rotation, and a caller's own output off the 8 bytes of a store goes to the generic kernel
+    if (f.D != 64 && f.D != 128 && (f.rope_q || (uintptr_t)f.o % 8 != 0)) return false;
     if (f.L < 1 || f.S < 1 || !(f.scale > 0.0f)) return false;
     if (f.L >= (1LL << 30) || f.S >= (1LL << 30)) return false;  // 32-bit row indices
     const int64_t strides[] = {f.q_sb, f.q_sh, f.q_sl, f.k_sb, f.k_sh, f.k_ss, f.v_sb, f.v_sh, f.v_ss};

@@ -97,3 +97,16 @@ def test_dropout(dev):
     assert_close(out32, ref, torch.float16, "out32", out_dtype=torch.float32)
     for name, got, want in zip(("dq", "dk", "dv"), grads, refs):
         assert_close(got, want, torch.bfloat16, name, out_dtype=torch.float32)
+
+
+@pytest.mark.parametrize("offset", [0, 1, 4])
+def test_callers_output_off_the_stores_alignment(dev, offset):
+    from test_zz_no_alloc import noalloc
+
+    B, H, L, D = 1, 2, 40, 80
+    q, k, v = (randn((B, H, L, D), 70 + i, torch.float16).to(dev) for i in range(3))
+    flat = torch.zeros(B * H * L * D + offset, dtype=torch.float16, device=dev)
+    out = flat[offset:].view(B, H, L, D)
+    assert noalloc(q, k, v, causal=True, out=out) == 0
+    assert _C.last_launch().startswith("generic" if offset % 4 else "prefill f16 D=80"), _C.last_launch()
+    assert_close(out, oracle_forward(q.cpu(), k.cpu(), v.cpu(), is_causal=True), torch.float16, f"offset {offset}")
