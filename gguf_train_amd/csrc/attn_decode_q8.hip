@@ -39,6 +39,7 @@
 #include "attn_common.h"
 #include "decode_merge.h"
 #include "gt_internal.h"
+#include "q8_tile.h"
 
 #include <algorithm>
 #include <cmath>
@@ -246,7 +247,7 @@ __global__ __launch_bounds__(256, 2) void decode_q8_lds_kernel(DecodeArgs a) {
 #pragma unroll
         for (int j = 0; j < NL; ++j) {
             const bool spare = TAIL != 0 && j == NL - 1 && lane >= TAIL;
-            const uint32_t off = min(t0 + 1024u * j + (spare ? 0u : 16u * lane), last16);
+            const uint32_t off = gtq8::read_at(t0 + 1024u * j + (spare ? 0u : 16u * lane), last16);
             rk[j] = __builtin_nontemporal_load((const u32x4_a4 *)(kbase + off));
             rv[j] = __builtin_nontemporal_load((const u32x4_a4 *)(vbase + off));
         }
@@ -257,15 +258,15 @@ __global__ __launch_bounds__(256, 2) void decode_q8_lds_kernel(DecodeArgs a) {
     };
     auto stage = [&](int step) {
         const uint32_t t0 = (uint32_t)(kbeg + step * kStep + 32 * w) * RB;
-        if ((last16 & 15) != 0 && t0 + TB > last16 + 16) {
+        if (gtq8::ends_inside_piece(t0, TB, last16)) {
             // the piece that straddles the end of the slice was read from last16 (t0 is a multiple
             // of 16, the slice's size here is not)
 #pragma unroll
             for (int j = 0; j < NL; ++j) {
-                const uint32_t off = t0 + 1024u * j + 16u * lane;
-                if (off > last16 && off < last16 + 16) {
-                    rk[j] = shifted(rk[j], (off - last16) / 4);
-                    rv[j] = shifted(rv[j], (off - last16) / 4);
+                const uint32_t early = gtq8::dwords_early(t0 + 1024u * j + 16u * lane, last16);
+                if (early) {
+                    rk[j] = shifted(rk[j], early);
+                    rv[j] = shifted(rv[j], early);
                 }
             }
         }
