@@ -344,18 +344,11 @@ __global__ __launch_bounds__(256) void kv_append_vec_kernel(KvAppendVec a) {
     const I n8 = (I)a.n8;
     if (a.pos_next && blockIdx.x == 0 && blockIdx.y == 0)
         for (int b = threadIdx.x; b < a.B; b += 256) a.pos_next[b] = pos[b] + T;
-    const I i = (I)blockIdx.x * 256 + (I)threadIdx.x;
-    const bool live = i < n8;
-    const I ic = live ? i : 0;
-    const int per = D / 8, half = n_dims / 2;
-    const I r = ic / per;  // source row (b, h, t)
-    const int j = (int)(ic - r * per);
-    const I bh = r / T;
-    const int t = (int)(r - bh * T);
-    const I b = bh / Hkv;
-    const int h = (int)(bh - b * Hkv);
-    const int d0 = 8 * j;
-    const bool rotated = d0 < n_dims;
+    const KvAppendThread<I> th((I)blockIdx.x * 256 + (I)threadIdx.x, n8, D, Hkv, T);
+    const bool live = th.live;
+    const I b = th.b;
+    const int h = th.h, t = th.t, d0 = th.d0, half = n_dims / 2;
+    const bool rotated = th.rotates(n_dims);
     const bool lo_chunk = d0 < half;  // NeoX: the whole chunk is on one side of half
     const int64_t srow = b * s_sb + h * s_sh + t * s_st;
     float v[8], w[8];
@@ -363,21 +356,18 @@ __global__ __launch_bounds__(256) void kv_append_vec_kernel(KvAppendVec a) {
     if (rotated && neox) load8<SDT>(src, srow + (lo_chunk ? d0 + half : d0 - half), w);
     const int32_t p0 = pos[b];
     __shared__ float2 s_cs[kRopeInlineEntries];
-    const I r0 = (I)blockIdx.x * 256 / per;  // the workgroup's first row
+    const KvAngleRows<I> ang(blockIdx.x, n8, D, Hkv, T);
     if (n_dims && !a.table) {
         // the rows' angles: one set per sequence for a single token, else one per row
-        const I rl = min((I)blockIdx.x * 256 + 255, n8 - 1) / per;
-        const I b0 = r0 / Hkv;  // (T == 1: the first sequence)
-        const int n = (int)(T == 1 ? rl / Hkv - b0 + 1 : rl - r0 + 1) * half;
-        for (int e = threadIdx.x; e < n; e += 256) {
+        for (int e = threadIdx.x; e < ang.count * half; e += 256) {
             const int er = e / half;
             I eb;
             int et = 0;
             if (T == 1) {
-                eb = b0 + er;
+                eb = ang.b0 + er;
             } else {
-                const I ebh = (r0 + er) / T;
-                et = (int)(r0 + er - ebh * T);
+                const I ebh = (ang.r0 + er) / T;
+                et = (int)(ang.r0 + er - ebh * T);
                 eb = ebh / Hkv;
             }
             s_cs[e] = rope_cos_sin(rope_theta(pos[eb] + et, e - er * half, a.theta_scale), a.freq_scale);
@@ -389,7 +379,7 @@ __global__ __launch_bounds__(256) void kv_append_vec_kernel(KvAppendVec a) {
         const int first = neox ? (lo_chunk ? d0 : d0 - half) : d0 >> 1, np = neox ? 8 : 4;
         float2 cs8[8];
         const float2 *tab = a.table ? a.table + ((int64_t)b * T + t) * half
-                                    : s_cs + (int)(T == 1 ? b - r0 / Hkv : r - r0) * half;
+                                    : s_cs + ang.place(th, T) * half;
 #pragma unroll
         for (int e = 0; e < 8; ++e)
             if (e < np) cs8[e] = tab[first + e];
@@ -420,7 +410,7 @@ __global__ __launch_bounds__(256) void kv_append_vec_kernel(KvAppendVec a) {
         const float id = d != 0.0f ? __fdiv_rn(1.0f, d) : 0.0f;
         if (!live) return;
         uint16_t *blk = (uint16_t *)((uint8_t *)dst + (row * (D / 32) + d0 / 32) * 34);  // 34 is even
-        const int part = j & 3;
+        const int part = (d0 / 8) & 3;
         if (part == 0) blk[0] = d_f32_to_f16(d);
 #pragma unroll
         for (int e = 0; e < 8; e += 2) {

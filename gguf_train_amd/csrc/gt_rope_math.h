@@ -10,6 +10,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include "rope_rows.h"
+
 // Angle of pair i at position p: theta_i is the float32 chain of i products (one rounding each), as
 // ggml forms it; theta_{i+1} = theta_i * theta_scale continues it.  The chain's length differs between
 // the lanes, so it is walked 8, 4, 2 and 1 products at a time: one product per iteration spends most of a
@@ -31,16 +33,6 @@ __device__ inline float2 rope_cos_sin(float theta, float freq_scale) {
     sincosf(freq_scale * theta, &sn, &cs);
     return make_float2(cs, sn);
 }
-// Threads (of a kernel that rotates up to 8 elements each) up to which a workgroup forms its rows' angles
-// itself, into LDS; more of them share a table made by a launch before, since a prompt's workgroups
-// would repeat each angle for every head.  A decode step's rows then take one launch: RoPE of fp16 B4
-// H32 D128 3.2 + 5.2 -> 3.9 us.  (Every thread forming its own 8 angles took 7.6 us: one accurate
-// sincosf after the other.)
-constexpr int64_t kRopeInlineThreads = 65536;
-constexpr int kRopeInlineMaxDim = 256;  // head size up to which the angles of a workgroup's rows fit
-// Angles of a 256-thread workgroup's rows: 8 elements per thread are 2048 / D rows, and one more at
-// either end when rows straddle workgroups.
-constexpr int kRopeInlineEntries = 1024 + kRopeInlineMaxDim;
 
 __device__ inline float rope_rot_lo(float lo, float hi, float2 cs) {
     float r = __fmaf_rn(lo, cs.x, -(hi * cs.y));
