@@ -16,6 +16,7 @@
 #include "gt_rope_math.h"
 
 #include <cmath>
+#include <type_traits>
 
 namespace {
 
@@ -320,7 +321,8 @@ __device__ inline void load8(const void *base, int64_t e0, float *v) {
 // pos_next, the first workgroup writes the lengths after the append.  A decode step's append is a chain of
 // latencies (position, angles, rows), not bandwidth: I, the type that indexes threads and rows, is int32_t
 // wherever they fit (a 64-bit division is about 100 dependent instructions), and the source rows are
-// loaded before the angles are formed (Q8_0, B4 Hkv8 T1 D128 with RoPE: 8.6 -> 6.5 us).
+// loaded before the angles are formed (Q8_0, B4 Hkv8 T1 D128 with RoPE: 8.6 -> 6.5 us; with the angles
+// kept in registers, on another day, 7.3 -> 5.9, and at T500 10.6 -> 7.7).
 struct KvAppendVec {
     const void *src[2];
     void *dst[2];
@@ -374,28 +376,40 @@ __global__ __launch_bounds__(256) void kv_append_vec_kernel(KvAppendVec a) {
         }
         __syncthreads();
     }
-    if (rotated) {
-        // the chunk's pairs in order: first, first + 1, ...
-        const int first = neox ? (lo_chunk ? d0 : d0 - half) : d0 >> 1, np = neox ? 8 : 4;
-        float2 cs8[8];
-        const float2 *tab = a.table ? a.table + ((int64_t)b * T + t) * half
-                                    : s_cs + ang.place(th, T) * half;
+    // The chunk's pairs in order: first, first + 1, ...  One copy of the rotation for each pairing and each
+    // place of the angles: with the pairing chosen per element the angles were indexed at run time, so they
+    // went through private memory, and a pointer to either place made every read of them a flat load.
+    auto rotate = [&](auto pairing, const float2 *tab) {
+        constexpr bool NEOX = decltype(pairing)::value;
+        constexpr int NP = NEOX ? 8 : 4;
+        const float2 *at = tab + (NEOX ? (lo_chunk ? d0 : d0 - half) : d0 >> 1);
+        float2 cs[8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
-            if (e < np) cs8[e] = tab[first + e];
+        for (int e = 0; e < NP; ++e) cs[e] = at[e];
         float rr[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-            const bool lo = neox ? lo_chunk : (e & 1) == 0;
-            const float other = neox ? w[e] : v[e ^ 1];
-            const float2 cs = neox ? cs8[e] : cs8[e >> 1];
-            float x = lo ? rope_rot_lo(v[e], other, cs) : rope_rot_hi(other, v[e], cs);
-            if constexpr (SDT == GT_F16) x = d_f16_to_f32(d_f32_to_f16(x));
+            const bool lo = NEOX ? lo_chunk : (e & 1) == 0;
+            const float own = v[e], other = NEOX ? w[e] : v[e ^ 1];
+            const float2 c = NEOX ? cs[e] : cs[e >> 1];
+            float x = lo ? rope_rot_lo(own, other, c) : rope_rot_hi(other, own, c);
+            if constexpr (SDT == GT_F16) x = d_f16_to_f32_fast(d_f32_to_f16(x));
             else if constexpr (SDT == GT_BF16) x = u2f((uint32_t)d_f32_to_bf16(x) << 16);
             rr[e] = x;
         }
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] = rr[e];
+    };
+    if (rotated) {
+        if (a.table) {
+            const float2 *tab = a.table + ((int64_t)b * T + t) * half;
+            if (neox) rotate(std::true_type{}, tab);
+            else rotate(std::false_type{}, tab);
+        } else {
+            const float2 *tab = s_cs + ang.place(th, T) * half;
+            if (neox) rotate(std::true_type{}, tab);
+            else rotate(std::false_type{}, tab);
+        }
     }
     const int64_t row = ((int64_t)b * Hkv + h) * cap + p0 + t;
     if constexpr (DDT == GT_Q8_0) {
