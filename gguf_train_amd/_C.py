@@ -253,18 +253,27 @@ def _load_bridge():
     """The CPython module that lends tensors to the library (built with it, and checked like it)."""
     import torch  # noqa: F401  (its libraries first: the module links to them by name)
 
-    from ._srchash import bridge_hash
-
     try:
         from . import _gt_bridge
     except ImportError as e:
         raise ImportError(f"{_PKG_DIR / '_gt_bridge.so'} is not built or does not load ({e}); build it with "
                           "`python gguf_train_amd/_build.py`") from e
-    want = bridge_hash()
-    if want is not None and _gt_bridge.SOURCE_HASH != want:
-        raise ImportError(f"{_gt_bridge.__file__} was built from other sources; rebuild it with "
-                          "`python gguf_train_amd/_build.py`")
+    _check_bridge(_gt_bridge)
     return _gt_bridge
+
+
+def _check_bridge(module) -> None:
+    """Refuses a bridge built from other sources, or for another PyTorch or Python: it reads their objects
+    inline, so it would load and misread them."""
+    from ._srchash import bridge_hash, bridge_target
+
+    want = bridge_hash()
+    if want is not None and module.SOURCE_HASH != want:
+        raise ImportError(f"{module.__file__} was built from other sources; rebuild it with "
+                          "`python gguf_train_amd/_build.py`")
+    if module.BUILT_FOR != bridge_target():
+        raise ImportError(f"{module.__file__} was built for {module.BUILT_FOR}, this is {bridge_target()}; rebuild it "
+                          "with `python gguf_train_amd/_build.py`")
 
 
 bridge = _load_bridge()

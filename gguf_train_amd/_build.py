@@ -106,11 +106,11 @@ def build_bridge() -> Path:
     torch_dir = Path(find_spec("torch").origin).resolve().parent
     inc, lib = torch_dir / "include", torch_dir / "lib"
     obj, tmp = OBJ_DIR / "torch_bridge.cpp.o", BRIDGE_PATH.with_suffix(".so.tmp")
-    digest = _srchash().bridge_hash(PKG_DIR)
+    digest, target = _srchash().bridge_hash(PKG_DIR), _srchash().bridge_target()
     OBJ_DIR.mkdir(exist_ok=True)
     for cmd in (
         ["g++", "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-Wall", f'-DGT_BRIDGE_HASH="{digest}"',
-         f"-I{sysconfig.get_paths()['include']}", f"-isystem{inc}", f"-isystem{inc}/torch/csrc/api/include", "-c",
+         f'-DGT_BRIDGE_TARGET="{target}"', f"-I{sysconfig.get_paths()['include']}", f"-isystem{inc}", f"-isystem{inc}/torch/csrc/api/include", "-c",
          str(BRIDGE_SRC), "-o", str(obj)],
         ["g++", "-shared", "-o", str(tmp), str(obj), f"-L{PKG_DIR}", "-l:libgt_attn.so", f"-L{lib}", "-ltorch_python",
          "-ltorch_cpu", "-lc10", "-Wl,-rpath,$ORIGIN"],

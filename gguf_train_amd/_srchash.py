@@ -40,3 +40,19 @@ def bridge_hash(pkg_dir: Path = PKG_DIR) -> str | None:
     if not all(p.is_file() for p in files):
         return None
     return hashlib.sha256(b"\0".join(p.read_bytes() for p in files)).hexdigest()
+
+
+def bridge_target() -> str:
+    """What the PyTorch bridge is compiled against and reads inline (at::Tensor, CPython objects): the
+    interpreter's ABI and PyTorch's version and revision.  Read from PyTorch's version file, so that the
+    build need not import PyTorch."""
+    import importlib.util
+    import sys
+    import sysconfig
+
+    path = Path(importlib.util.find_spec("torch").origin).parent / "version.py"
+    spec = importlib.util.spec_from_file_location("_gt_torch_version", path)
+    version = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(version)
+    python = ".".join(map(str, sys.version_info[:3]))
+    return f"python {python} {sysconfig.get_config_var('SOABI')}, torch {version.__version__} {version.git_version}"

@@ -20,6 +20,9 @@
 #ifndef GT_BRIDGE_HASH
 #define GT_BRIDGE_HASH ""
 #endif
+#ifndef GT_BRIDGE_TARGET
+#define GT_BRIDGE_TARGET ""
+#endif
 
 namespace {
 
@@ -241,7 +244,8 @@ PyMODINIT_FUNC PyInit__gt_bridge(void) {
     if (!m) return nullptr;
     Py_INCREF(&HandleType);
     if (PyModule_AddObject(m, "Handle", (PyObject *)&HandleType) < 0 ||
-        PyModule_AddStringConstant(m, "SOURCE_HASH", GT_BRIDGE_HASH) < 0) {
+        PyModule_AddStringConstant(m, "SOURCE_HASH", GT_BRIDGE_HASH) < 0 ||
+        PyModule_AddStringConstant(m, "BUILT_FOR", GT_BRIDGE_TARGET) < 0) {
         Py_DECREF(m);
         return nullptr;
     }
