@@ -190,9 +190,11 @@ hipError_t launch_attn_prefill(const AttnFwdArgs &a, int cd, hipStream_t s);
 hipError_t launch_prefill_heads(const AttnFwdArgs &a, int cd, int nq, int order, int64_t grid, hipStream_t s);  // D = 80, 96
 int attn_prefill_key_tile(const AttnFwdArgs &f);  // keys per tile of the half-precision kernel
 // Fills t.cls and t.bits from a mask of `batches` (L, S) planes; kind 0 bool bytes, 1 float16, 2
-// bfloat16, 3 float32; copy: float32 values of the half-precision kinds' kMaskTileValues tiles.
+// bfloat16, 3 float32; causal: tiles above the diagonal are not looked at; copy: float32 values of the
+// half-precision kinds' kMaskTileValues tiles.
 hipError_t launch_attn_mask_tiles(int kind, const void *mask, int64_t batches, int64_t sb, int64_t sl, int64_t ss,
-                                  int64_t L, int64_t S, int bn, const AttnMaskTiles &t, float *copy, hipStream_t s);
+                                  int64_t L, int64_t S, int bn, int causal, const AttnMaskTiles &t, float *copy,
+                                  hipStream_t s);
 bool attn_prefill_asm_supported(const AttnFwdArgs &f, int cd);
 bool attn_prefill_f32_split(const AttnFwdArgs &f, int cd);  // float32: the small-grid kernel
 hipError_t launch_attn_prefill_asm(const AttnFwdArgs &a, hipStream_t s);

@@ -294,15 +294,18 @@ __global__ __launch_bounds__(64 * nw_of<D>(), DROP && (MASK == 1 || MASK == 2 ||
         vofs_n[n] = (uint32_t)lrow_n[n] * v_row + lcol_n[n];
     }
     const float *mrow = MROW ? (const float *)a.mask + b * a.m_sb + h * a.m_sh : nullptr;
-    // MTILE: bits of the keys of the step to come, one word per 32 keys of this lane's row
+    // MTILE: the list's entry of the step to come, and the bits of its keys, one word per 32 keys of this
+    // lane's row
+    static_assert(!MTILE || NST == 2, "one step to come");
+    int nent = 0;
     uint32_t nbits[MTILE ? NKB : 1];
     auto issue = [&](int step) {
         int kt = step < na ? step : step - na;
         const int st = step % NST;
         if constexpr (MTILE) {
-            const int e = entry(step);
-            kt = e & 0x3fff;
-            if (e >> 14 == kMaskTileBits) {
+            nent = entry(step);
+            kt = nent & 0x3fff;
+            if (nent >> 14 == kMaskTileBits) {
                 const int row = min((step < na ? qa : qb) * BM + 32 * w + lrow, L - 1);
                 const uint32_t *wd = a.mt.bits + (mtb * L + row) * a.mt.words;
 #pragma unroll
@@ -399,7 +402,7 @@ __global__ __launch_bounds__(64 * nw_of<D>(), DROP && (MASK == 1 || MASK == 2 ||
         const int64_t mrb = MVEC ? b * a.m_sb + h * a.m_sh + (int64_t)min(lq, L - 1) * a.m_sl : 0;
 
         for (int j = 0; j < ntiles; ++j, ++step) {
-            const int ent = MTILE ? entry(step) : j;
+            const int ent = MTILE ? nent : j;
             const int k0 = (MTILE ? ent & 0x3fff : j) * BN, mcls = MTILE ? ent >> 14 : 0;
             // Tile `step` is complete once at most the loads of the tiles issued after it are
             // outstanding (vector memory loads complete in order); the barrier then makes every
@@ -434,34 +437,71 @@ __global__ __launch_bounds__(64 * nw_of<D>(), DROP && (MASK == 1 || MASK == 2 ||
                     }
             }
 
+            // MTILE, tiles with other values: the mask's loads land during S = K.Q^T.  With two 32-key blocks
+            // there are registers for them beside the scores; with four (head size 64) such tiles have a
+            // product of their own, which keeps those registers out of the other tiles' way.  (After S, four
+            // loads at a time, they took a round trip per block: fp16 B4 H32 L=S=2048 D128 causal with
+            // float32 values 268 us, bf16 B8 H16 L=S=1024 D64 69.)
+            const float *mtrow = MTILE ? (const float *)a.mask + mtb * a.m_sb + (int64_t)min(lq, L - 1) * a.m_sl : nullptr;
+            f32x4 mtv[MTILE && NKB == 2 ? NKB : 1][4];
+            auto mt_load = [&](f32x4(*x)[4]) {  // (a copy's row pitch covers whole 4-key groups)
+#pragma unroll
+                for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+                    for (int g = 0; g < 4; ++g)
+                        x[kb][g] = *(const f32x4 *)(mtrow + min(k0 + 32 * kb + 8 * g + 4 * half, (S - 1) / 4 * 4));
+            };
+            if constexpr (MTILE && NKB == 2) {
+                if (mcls == kMaskTileValues) mt_load(mtv);
+            }
+
             // (causal) a wavefront whose rows all precede this tile still runs it: every score
             // is masked to -inf and p = 0; skipping it makes the compiler copy O on every tile
             // ---- S^T = K . Q^T ----
             // MROW: the key-padding row enters as the accumulator's initial value (mask / scale,
             // the raw-score units of the accumulator), so S^T = K.Q^T + mask costs no VALU add
             f32x16 s[NKB];
+            auto scores = [&]() {
 #pragma unroll
-            for (int kb = 0; kb < NKB; ++kb) {
-                V8 kf[DT];
+                for (int kb = 0; kb < NKB; ++kb) {
+                    V8 kf[DT];
 #pragma unroll
-                for (int t = 0; t < DT; ++t) kf[t] = *(const V8 *)&cK[kofs[t] + 32 * kb * PD];
-                if constexpr (MROW) {
+                    for (int t = 0; t < DT; ++t) kf[t] = *(const V8 *)&cK[kofs[t] + 32 * kb * PD];
+                    if constexpr (MROW) {
 #pragma unroll
-                    for (int g = 0; g < 4; ++g) {
-                        const f32x4 mv4 = *(const f32x4 *)&sMk[step % NST][32 * kb + 8 * g + 4 * half];
+                        for (int g = 0; g < 4; ++g) {
+                            const f32x4 mv4 = *(const f32x4 *)&sMk[step % NST][32 * kb + 8 * g + 4 * half];
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) s[kb][4 * g + e] = mv4[e] * inv_scale;
+                            for (int e = 0; e < 4; ++e) s[kb][4 * g + e] = mv4[e] * inv_scale;
+                        }
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < 16; ++i) s[kb][i] = 0.0f;
                     }
-                } else {
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) s[kb][i] = 0.0f;
+                    for (int t = 0; t < DT; ++t) s[kb] = M::mma(kf[t], qf[t], s[kb]);
                 }
-#pragma unroll
-                for (int t = 0; t < DT; ++t) s[kb] = M::mma(kf[t], qf[t], s[kb]);
-            }
-
+            };
             // the next tile's loads into the stage every wavefront finished with before the barrier
-            if (step + NST - 1 < total) issue(step + NST - 1);
+            auto prefetch = [&]() {
+                if (step + NST - 1 < total) issue(step + NST - 1);
+            };
+            auto add_values = [&](f32x4(*x)[4]) {
+#pragma unroll
+                for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) s[kb][i] = fmaf(x[kb][i / 4][i % 4], inv_scale, s[kb][i]);
+            };
+            if (MTILE && NKB > 2 && mcls == kMaskTileValues) {
+                f32x4 x[NKB][4];
+                mt_load(x);
+                scores();
+                prefetch();
+                add_values(x);
+            } else {
+                scores();
+                prefetch();
+            }
 
             // ---- masks: s[kb][i] is (key = k0 + 32kb + 8(i/4) + 4half + i%4, query = lq) ----
             const bool edge = k0 + BN > nkv || (CAUSAL && k0 + BN - 1 > wq0 + qpos);
@@ -473,18 +513,9 @@ __global__ __launch_bounds__(64 * nw_of<D>(), DROP && (MASK == 1 || MASK == 2 ||
 #pragma unroll
                         for (int i = 0; i < 16; ++i)
                             s[kb][i] = (mbits[kb] >> (8 * (i / 4) + (i % 4))) & 1u ? s[kb][i] : -INFINITY;
-                } else if (mcls == kMaskTileValues) {
-                    const float *mv = (const float *)a.mask + mtb * a.m_sb + (int64_t)min(lq, L - 1) * a.m_sl;
-#pragma unroll
-                    for (int kb = 0; kb < NKB; ++kb) {
-#pragma unroll
-                        for (int g = 0; g < 4; ++g) {
-                            const f32x4 x = *(const f32x4 *)(mv + min(k0 + 32 * kb + 8 * g + 4 * half, (S - 1) / 4 * 4));
-#pragma unroll
-                            for (int e = 0; e < 4; ++e) s[kb][4 * g + e] = fmaf(x[e], inv_scale, s[kb][4 * g + e]);
-                        }
-                        __builtin_amdgcn_sched_barrier(0);  // 4 loads in flight: 16 would spill at head size 64
-                    }
+                }
+                if constexpr (NKB == 2) {
+                    if (mcls == kMaskTileValues) add_values(mtv);
                 }
             }
             if ((MASK != 0 && !MROW && !MTILE) || edge) {

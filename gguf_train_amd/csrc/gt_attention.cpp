@@ -169,7 +169,7 @@ bool stage_mask(const gt_tensor *mask, int dev, int cd, AttnFwdArgs &a, Temps &t
 
 // The mask of a half-precision forward as tile classes (attn_mask_tiles.hip): one that varies along
 // the query rows and is shared by the heads, on the device in bool, float16, bfloat16 or float32.  The
-// pass over the mask and the list at the start of each workgroup cost about 8 us together, and a tile's
+// pass over the mask and the list at the start of each workgroup cost about 6 us together, and a tile's
 // mask work saved about 1 us of a workgroup's walk, so the line is a number of key tiles: 8 for bool and
 // float32 masks (band, GPU time with the mask as given against tile classes: D64 B2 H16 L128 S512 18.2
 // against 21.7 us, S1024 33.0 against 28.5; D128 B4 H32 L256 S512 27.3 against 25.7, S1024 47.1 against
@@ -177,6 +177,14 @@ bool stage_mask(const gt_tensor *mask, int dev, int cd, AttnFwdArgs &a, Temps &t
 // B2 H16 L128 S384 20.1 against 20.4, S512 23.9 against 22.2; D128 B4 H32 L256 S256 21.6 against 19.8,
 // S1024 54.8 against 37.9).  float32 masks need the 4-key alignment of mode 6 (tiles with other values
 // than 0 and -inf are read in place).  Call with q, k, v and the options of `a` final.
+// What the tiles hold is not known here.  Where every one holds other values, half-precision masks lose
+// nothing (their pass replaces the conversion's: D64 B2 H16 L128 S512 fp16 35 -> 25 us, bf16 B8 H16
+// L=S=1024 causal 60.7 -> 61.9) and float32 ones the pass: nothing to see without the causal mask (D128 B4
+// H32/8 L500 S1500 fp16 119 -> 84), 5 to 12 us with it, when the mask as given took the same tile order
+// (D128 B4 H32 L=S=2048 fp16 230 -> 242, bf16 259 -> 261; B1 H32/8 L=S=4000 fp16 201 -> 220, bf16 232 ->
+// 233; D64 B8 H16 L=S=1024 fp16 52 -> 59, bf16 51 -> 60).  The same calls with a band or a finite blocked
+// value gain more (fp16: 226 -> 174 and 180; 199 -> 160 and 161; 52 -> 37 and 41), and a window or
+// documents skip most tiles.
 // 1: staged, 0: not of this kind, -1: error.
 int stage_mask_tiles(const gt_tensor *mask, int dev, int cd, AttnFwdArgs &a, gt_scratch &mem) {
     if (!mask || (cd != GT_F16 && cd != GT_BF16) || a.dropout || a.rope_q || a.L <= 1 || a.S < 4) return 0;
@@ -214,7 +222,7 @@ int stage_mask_tiles(const gt_tensor *mask, int dev, int cd, AttnFwdArgs &a, gt_
     t.words = (int)words;
     t.batched = batches > 1;
     float *values = (float *)(p + bits + cls);
-    if (!gt_hip_check(launch_attn_mask_tiles(kind, gt_data(mask), batches, sb, sl, ss, a.L, a.S, bn, t, values, gt_stream()),
+    if (!gt_hip_check(launch_attn_mask_tiles(kind, gt_data(mask), batches, sb, sl, ss, a.L, a.S, bn, a.causal, t, values, gt_stream()),
                       "flash_attention: mask tiles kernel"))
         return -1;
     a.mt = t;
@@ -296,7 +304,7 @@ std::string decode_note(const char *kind, const DecodeArgs &da, int max_tile) {
 std::string prefill_note(const AttnFwdArgs &a, int cd) {
     return std::string(attn_prefill_asm_supported(a, cd) ? "prefill pipelined " : "prefill ") + dtype_tag(cd) + " D=" + std::to_string(a.D) + " B=" + std::to_string(a.B) +
            " H=" + std::to_string(a.H) + " L=" + std::to_string(a.L) + " S=" + std::to_string(a.S) +
-           (attn_prefill_f32_split(a, cd) ? " split" : "");
+           (attn_prefill_f32_split(a, cd) ? " split" : "") + (a.mt.cls ? " mask_tiles" : "");
 }
 
 bool dispatch_forward(const AttnFwdArgs &a, int cd, int dev) {
