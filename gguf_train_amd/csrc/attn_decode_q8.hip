@@ -42,6 +42,7 @@
 #include "q8_tile.h"
 
 #include <algorithm>
+#include <cfloat>
 #include <cmath>
 #include <map>
 #include <mutex>
@@ -359,7 +360,14 @@ __global__ __launch_bounds__(256, 2) void decode_q8_lds_kernel(DecodeArgs a) {
                 if (MASK != 0) {
                     const int64_t mi = mrow + (int64_t)min(key, S - 1) * f.m_ss;
                     if (MASK == 1) blocked = blocked || !((const uint8_t *)f.mask)[mi];
-                    else x = fmaf(((const float *)f.mask)[mi], kLog2e, x);
+                    else if constexpr (!WIDE) x = fmaf(((const float *)f.mask)[mi], kLog2e, x);
+                    else {
+                        // a finite value below -FLT_MAX / log2(e) (a mask of the type's lowest value) stays above
+                        // -inf: a sequence with no other keys averages their values, as the generic kernel has it
+                        const float mv = ((const float *)f.mask)[mi];
+                        x = fmaf(mv, kLog2e, x);
+                        x = x == -INFINITY && mv != -INFINITY ? -FLT_MAX : x;
+                    }
                 }
                 x = blocked ? -INFINITY : x;
                 sc[kb][i] = x;
