@@ -146,7 +146,8 @@ PyObject *borrow(PyObject *, PyObject *arg) {
 }
 
 // borrow_q8(data, shape) -> Handle on the Q8_0 blocks in the contiguous uint8 device tensor `data`, a
-// dense tensor of the logical shape; None when data is another kind of tensor.
+// dense tensor of the logical shape; None when data is another kind of tensor or the shape holds other
+// than integers.
 PyObject *borrow_q8(PyObject *, PyObject *const *args, Py_ssize_t n) {
     if (n != 2 || !THPVariable_Check(args[0]) || !PyTuple_Check(args[1])) {
         PyErr_SetString(PyExc_TypeError, "borrow_q8: expected (tensor, tuple)");
@@ -157,7 +158,10 @@ PyObject *borrow_q8(PyObject *, PyObject *const *args, Py_ssize_t n) {
     int64_t shape[GT_MAX_DIMS + 1], strides[GT_MAX_DIMS + 1];
     for (Py_ssize_t i = 0; i < ndim; ++i) {
         shape[i] = PyLong_AsLongLong(PyTuple_GET_ITEM(args[1], i));
-        if (shape[i] == -1 && PyErr_Occurred()) return nullptr;
+        if (shape[i] == -1 && PyErr_Occurred()) {  // a float, say: the caller's path takes what int() takes
+            PyErr_Clear();
+            Py_RETURN_NONE;
+        }
     }
     int64_t acc = 1;
     for (Py_ssize_t i = ndim - 1; i >= 0; --i) {
