@@ -120,7 +120,7 @@ class MultiheadAttention(nn.Module):
         S = key.shape[1]
         H, D = self.num_heads, self.head_dim
         # (B, L, H, D) memory viewed as (B, H, L, D): the kernels read these strides directly
-        if same and self._qkv_same:
+        if same and self._qkv_same and self._packed_rows_fit(L, E, self.in_proj_weight.element_size()):
             # one product for q, k and v, and one each for their gradients, with no input gradients to add
             # and no weight gradients to concatenate (float32 B8 L256 E512 H8, forward and backward: 38 -> 24
             # launches a pass, the products and copies 42 us less)
@@ -202,6 +202,13 @@ class MultiheadAttention(nn.Module):
             if attn_weights is not None:
                 attn_weights = attn_weights.squeeze(0)
         return out, attn_weights
+
+    @staticmethod
+    def _packed_rows_fit(L: int, E: int, nbytes: int) -> bool:
+        """Whether rows of q, k and v at a stride of 3E keep a head's span within the 32-bit byte offsets
+        of the MFMA kernels; past them a call takes the generic kernels, which rows of E reach at three
+        times the length."""
+        return L * 3 * E * nbytes <= 0xFFFFFFFF
 
     @staticmethod
     def _additive_mask(mask, dtype, name: str):
