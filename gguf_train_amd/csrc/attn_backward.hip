@@ -836,7 +836,7 @@ bool bwd_f32_small(const AttnFwdArgs &f) {
 
 bool bwd_f32_supported(const AttnBwdArgs &a) {
     const AttnFwdArgs &f = a.f;
-    if (f.D != f.Dv || (f.D != 64 && f.D != 128) || f.kv_len || f.q_pos) return false;
+    if (f.D != f.Dv || (f.D != 64 && f.D != 128) || f.kv_len) return false;
     const int mode = attn_mask_mode(f);
     // as the forward: fewer than 16 query rows take the small-grid kernels or the generic ones
     if ((f.L < 16 && !bwd_f32_small(f)) || f.L < 1 || f.S < 1 || !(f.scale > 0.0f) || !f.o || !f.lse)

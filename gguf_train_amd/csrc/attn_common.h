@@ -49,12 +49,11 @@ struct AttnFwdArgs {
     int causal;
     int mask_bool;
     int out_dtype;  // gt_dtype of o
-    // Per-sequence key lengths and query positions (a KV cache; both null for the reference
-    // operator): key s of batch b is present when s < kv_len[b], and the causal test is
-    // s <= q_pos[b] + l (null: s < S, and q_pos = 0, the reference's top-left alignment).
+    // Per-sequence key lengths (a KV cache; null for the reference operator): key s of batch b is present
+    // when s < kv_len[b] (null: s < S).  The causal test is s <= p + l: p = kv_len[b] - L with q_tail (the
+    // query rows are the sequence's last L keys), else 0, the reference's top-left alignment.
     const int32_t *kv_len;
-    const int32_t *q_pos;
-    int q_tail;  // the query rows are the sequence's last L keys: position kv_len[b] - L (q_pos null)
+    int q_tail;
     // RoPE of the queries (all D dims) applied as the prefill kernel loads them (null: none):
     // (cos, sin) of pair i of query row l at rope_q[l * D / 2 + i]; rope_neox: NeoX pairing.
     const void *rope_q;  // float2
@@ -84,7 +83,7 @@ inline int attn_mask_mode(const AttnFwdArgs &a) {
 
 __device__ inline int attn_kv_len(const AttnFwdArgs &a, int64_t b) { return a.kv_len ? a.kv_len[b] : (int)a.S; }
 __device__ inline int attn_q_pos(const AttnFwdArgs &a, int64_t b) {
-    return a.q_tail ? a.kv_len[b] - (int)a.L : a.q_pos ? a.q_pos[b] : 0;
+    return a.q_tail ? a.kv_len[b] - (int)a.L : 0;
 }
 // Wave priority by progress: 3, 2, 1, 0 for steps 0, 1, 2, 3 (mod 4) of a kernel's step loop.
 // Two workgroups resident on one CU share its SIMDs, and among waves of equal priority a SIMD

@@ -591,7 +591,9 @@ bool attn_decode_q8_supported(const AttnFwdArgs &f, int q_dtype) {
     if (decode_units(f.B, f.H, f.Hkv, kDecodeQ8MaxTile) > 65535) return false;
     const int64_t q16 = q_dtype == GT_F32 ? 4 : 8;  // query rows start 16-byte aligned
     if (f.q_sh % q16 != 0 || f.q_sb % q16 != 0 || (uintptr_t)f.q % 16 != 0) return false;
-    // K/V are whole dense Q8_0 tensors; rows are 4-byte aligned when the base is
+    // K/V are whole dense Q8_0 tensors.  The kernel's reads need 4-byte alignment; bases off 8 bytes keep the
+    // dequantizing path, which gt_flash_attention_noalloc refuses (allocations and the tensors of a GGUF
+    // file start at 32 bytes or more)
     for (const void *p : {f.k, f.v}) if ((uintptr_t)p % 8 != 0) return false;
     return true;
 }

@@ -78,7 +78,7 @@ bool asm_enabled() { return false; }
 bool attn_prefill_asm_supported(const AttnFwdArgs &f, int cd) {
     if (!asm_enabled()) return false;
     if (cd != GT_F16 || f.out_dtype != GT_F16 || f.D != 128 || f.Dv != 128) return false;
-    if (f.mask || f.dropout || f.rope_q || f.o32 || f.kv_len || f.q_pos) return false;
+    if (f.mask || f.dropout || f.rope_q || f.o32 || f.kv_len) return false;
     if (!(f.scale > 0.0f) || f.L < 1) return false;
     if (f.causal) {
         if (f.L != f.S || f.L % kRows != 0) return false;

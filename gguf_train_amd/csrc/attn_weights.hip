@@ -537,7 +537,7 @@ hipError_t launch_generic(const AttnFwdArgs &f, void *w, bool avg, hipStream_t s
 // `w` receives (B,H,L,S), or (B,L,S) when averaging over the heads.
 bool attn_weights_mfma(const AttnFwdArgs &f, int cd) {
     if ((cd != GT_F16 && cd != GT_BF16 && cd != GT_F32) || (f.D != 64 && f.D != 128) || f.out_dtype != cd) return false;
-    if (f.kv_len || f.q_pos || f.dropout || (uintptr_t)f.q % 16 != 0 || (uintptr_t)f.k % 16 != 0) return false;
+    if (f.kv_len || f.dropout || (uintptr_t)f.q % 16 != 0 || (uintptr_t)f.k % 16 != 0) return false;
     const int64_t rows = cd == GT_F32 ? 4 : 8;  // 16-byte rows
     for (int64_t st : {f.q_sb, f.q_sh, f.q_sl, f.k_sb, f.k_sh, f.k_ss})
         if (st % rows != 0) return false;

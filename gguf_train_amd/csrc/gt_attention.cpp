@@ -2,8 +2,8 @@
 // operand staging onto the device, kernel selection, and the Q8_0 codec entry points.
 //
 // gt_flash_attention keeps the contract of csrc/gt_ops_nn.cpp:2423-2525; the kernels it
-// dispatches to live in attn_generic.hip (any dtype/shape), attn_decode.hip (single-query
-// split-K over the KV length, fp16/bf16/Q8_0 K/V) and attn_prefill.hip (fp16/bf16 MFMA).
+// dispatches to live in attn_generic.hip (any dtype/shape), attn_decode.hip and attn_decode_q8.hip
+// (single-query split-K over the KV length) and attn_prefill.hip (fp16/bf16/float32 MFMA).
 
 #include "attn_common.h"
 #include "gt_internal.h"
@@ -289,8 +289,6 @@ bool decode_partials(DecodeArgs &da, int64_t units, int dev, gt_scratch &scratch
     return true;
 }
 
-// Picks the kernel for a staged forward: split-K decode for single-query rows, the MFMA
-// prefill kernel for fp16/bf16 with head size 64/128, the generic kernel otherwise.
 // Launch-log entry of a split-K decode launch.
 std::string decode_note(const char *kind, const DecodeArgs &da, int max_tile) {
     const AttnFwdArgs &a = da.f;
@@ -307,6 +305,8 @@ std::string prefill_note(const AttnFwdArgs &a, int cd) {
            (attn_prefill_f32_split(a, cd) ? " split" : "") + (a.mt.cls ? " mask_tiles" : "");
 }
 
+// Picks the kernel for a staged forward: split-K decode for single-query rows, the MFMA prefill kernels
+// (fp16/bf16: head sizes 64, 80, 96 and 128; float32: 64 and 128), the generic kernel otherwise.
 bool dispatch_forward(const AttnFwdArgs &a, int cd, int dev) {
     if (a.out_dtype == cd && !a.o32 && !a.dropout && attn_decode_supported(a, cd)) {
         DecodeArgs da{};
@@ -430,8 +430,9 @@ bool copies_rows(int cd, int64_t L, int64_t D, int64_t Dv) {
     return (cd == GT_F16 || cd == GT_BF16) && L > 1 && D == Dv && D > 64 && D < 128 && mfma_head(cd, D) == D;
 }
 
-// Float32 calls whose padded form the float32 MFMA kernels take (masks staged, dropout applied).
-bool f32_pads(const AttnFwdArgs &a) { return !a.kv_len && !a.q_pos; }
+// Float32 calls whose padded form the float32 MFMA kernels take: those without KV-cache lengths, whatever
+// their mask and dropout (the forward asks before its mask is staged).
+bool f32_pads(const AttnFwdArgs &a) { return !a.kv_len; }
 
 // A dense (d0, d1, d2, Dp) copy of the 4-D device tensor t (innermost contiguous, 2- or 4-byte
 // elements) whose dims past t's last are zero; kept in tmp.
@@ -1104,8 +1105,8 @@ extern "C" int gt_flash_attention_noalloc(const gt_tensor *q, const gt_tensor *k
     }
     const bool q8 = k->dtype == GT_Q8_0 || v->dtype == GT_Q8_0;
     if (q8 && !(k->dtype == GT_Q8_0 && v->dtype == GT_Q8_0 && q->dtype == GT_F16 && L == 1)) {
-        gt_set_error(std::string(who) + ": q8_0 k/v need float16 q with one query row (L = 1); other q8_0 "
-                     "calls dequantize, which allocates");
+        gt_set_error(std::string(who) + ": q8_0 k/v need float16 q with one query row (L = 1); more rows "
+                     "dequantize, which allocates, and other q dtypes are not taken here");
         return -1;
     }
     const int cd = q8 ? GT_F16 : q->dtype;
