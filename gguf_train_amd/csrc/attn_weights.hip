@@ -19,6 +19,7 @@
 // element's multiplier m (gt_philox.h); computed by the per-element kernel.
 
 #include "attn_common.h"
+#include "attn_weights_rule.h"
 #include "gt_internal.h"
 #include "mfma_util.h"
 
@@ -454,13 +455,6 @@ unsigned key_splits(int64_t grid, int64_t nkt, bool avg) {
     return (unsigned)std::max<int64_t>(1, std::min<int64_t>(nkt, (1024 + grid - 1) / grid));
 }
 
-// Averaged float32 weights whose heads are split over a workgroup's wavefronts (`grid`: workgroups of 128
-// query rows, nkt: 64-key tiles): while the unsplit grid has less than one workgroup for each of the 256
-// CUs.  From there on the SIMDs are busy either way, and Q and K are loaded by four times the workgroups
-// (D64 H8, key padding, unsplit against split: B8 L=S=256, 64 workgroups, 56.9 against 19.3 us; B4 L=S=512,
-// 128, 57.9 against 34.8; B8 L=S=512, 256, 61.6 against 66.8; B16, 512, 119.6 against 130.5).
-bool f32_heads_split(int64_t grid, int64_t nkt, int64_t H) { return H >= WQ && grid * nkt < 256; }
-
 template <typename T, int D, bool AVG>
 hipError_t launch_mfma(const AttnFwdArgs &f, void *w, hipStream_t st) {
     const int64_t nrb = (f.L + 32 * WQ - 1) / (32 * WQ);
@@ -491,7 +485,7 @@ hipError_t launch_mfma(const AttnFwdArgs &f, void *w, hipStream_t st) {
 template <int D, bool AVG>
 hipError_t launch_f32(const AttnFwdArgs &f, void *w, hipStream_t st) {
     int64_t nrb = (f.L + 32 * WQ - 1) / (32 * WQ);
-    const bool hs = AVG && f32_heads_split(nrb * f.B, (f.S + 63) / 64, f.H);
+    const bool hs = AVG && f32_heads_split(nrb * f.B, (f.S + 63) / 64, f.H, WQ);
     if (hs) nrb = (f.L + 31) / 32;
     const int64_t grid = nrb * (AVG ? f.B : f.B * f.H);
     if (grid > 0x7fffffffLL) return hipErrorInvalidConfiguration;

@@ -1,5 +1,5 @@
 """Averaged float32 weights of small grids: a workgroup's wavefronts take the heads in turn and add their
-tiles.  Grids on both sides of the rule (256 workgroups of 128 rows and 64 keys), head counts that are and
+tiles.  Grids on both sides of the rule (up to 128 workgroups of 128 rows and 64 keys), head counts that are and
 are not whole rounds of the four wavefronts, rows and keys that are not whole tiles, against the mean of
 the weights per head."""
 
@@ -15,6 +15,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("B,H,Hkv,L,S,D", [(1, 4, 4, 1, 5, 64), (2, 5, 5, 33, 64, 64), (1, 8, 2, 130, 257, 128), (3, 3, 3, 70, 66, 64),
+                                           (8, 9, 9, 100, 1000, 64), (8, 4, 4, 100, 1025, 64),
                                            (8, 9, 9, 100, 1985, 64), (8, 4, 4, 100, 2049, 64)])
 @pytest.mark.parametrize("causal,mkind", [(False, None), (True, "pad"), (False, "bool")])
 def test_average_is_the_mean_of_the_heads(dev, B, H, Hkv, L, S, D, causal, mkind):
