@@ -51,7 +51,11 @@ def test_masks_shared_by_the_heads(dev, dtype, D, L, S, batches, causal, kind, m
     # the same mask as a view with another layout
     wide = torch.zeros((*mask.shape[:-1], S + 3), dtype=mask.dtype, device=dev)
     wide[..., :S] = mask.to(dev)
-    assert torch.equal(g.flash_attention(q.to(dev), k.to(dev), v.to(dev), wide[..., :S], 0.0, causal), got) or mdtype == torch.float32
+    view = g.flash_attention(q.to(dev), k.to(dev), v.to(dev), wide[..., :S], 0.0, causal)
+    if mdtype == torch.float32:  # rows off the 4-key groups: read as given, in another order of operations
+        assert_close(view, want, dtype, f"{kind} view")
+    else:
+        assert torch.equal(view, got)
     turned = mask.to(dev).transpose(-1, -2).contiguous().transpose(-1, -2)
     assert_close(g.flash_attention(q.to(dev), k.to(dev), v.to(dev), turned, 0.0, causal), want, dtype, "turned")
 

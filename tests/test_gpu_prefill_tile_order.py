@@ -1,14 +1,17 @@
 """Every way the half-precision prefill deals query tiles to workgroups (pairs of tiles, single tiles
 heaviest first, single tiles folded, head by head), with heads that do and do not divide among the 8
-XCDs and odd tile counts, against the float64 oracle on a few heads; every row of every head is also
-checked to be written (the output buffer holds other calls' values before)."""
+XCDs and odd tile counts.  The output is the caller's own, NaN before the call, so a row that no
+workgroup writes shows; every head is compared with the float32 kernels, whose workgroups are dealt
+otherwise, and a few with the float64 oracle."""
 
 import pytest
 import torch
 
 import gguf_train_amd as g
+from gguf_train_amd import _C
 
 from _util import assert_close, oracle_forward, randn
+from test_zz_no_alloc import noalloc
 
 pytestmark = pytest.mark.gpu
 
@@ -37,10 +40,13 @@ def _order(causal, nq, heads):
 def test_every_tile_order(dev, dtype, B, H, Hkv, L, S, D, causal, order):
     assert _order(causal, (L + 127) // 128, B * H) == order
     q, k, v = (randn((B, h, n, D), i + L, dtype) for i, (h, n) in enumerate(((H, L), (Hkv, S), (Hkv, S))))
-    poison = torch.full((B, H, L, D), float("nan"), dtype=dtype, device=dev)
-    del poison  # its block is what the output gets next: rows nobody wrote would be NaN
-    got = g.flash_attention(q.to(dev), k.to(dev), v.to(dev), None, 0.0, causal)
-    assert torch.isfinite(got).all()
+    qd, kd, vd = (t.to(dev) for t in (q, k, v))
+    got = torch.full((B, H, L, D), float("nan"), dtype=dtype, device=dev)
+    assert noalloc(qd, kd, vd, None, 0.0, causal, got) == 0, _C.last_error()
+    assert _C.last_launch().startswith(f"prefill {'f16' if dtype == torch.float16 else 'bf16'} D={D} "), _C.last_launch()
+    every = g.flash_attention(qd.float(), kd.float(), vd.float(), None, 0.0, causal)
+    assert_close(got, every.double().cpu().numpy(), dtype, "every head")
+    assert torch.equal(g.flash_attention(qd, kd, vd, None, 0.0, causal), got)
     G = H // Hkv
     for b, h in {(0, 0), (B - 1, H - 1), (0, H // 2)}:
         kv = slice(h // G, h // G + 1)
