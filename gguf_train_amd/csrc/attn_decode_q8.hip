@@ -32,9 +32,9 @@
 // The products are exact and the sums float32, so only the summation order differs from
 // dequantizing to float32 and attending in float32, which is what these calls did before (two
 // dequantize passes, then the generic kernel for bf16 and the float32 decode kernel for float32):
-// B16 H32/8 S8192 D128 bf16 1399 -> 61 us (4.7 TB/s), float32 469 -> 65 us; B4 S3001 bf16 413 -> 18
-// us, float32 51 -> 18 us, of which most is the call itself.  Measured error of float32 queries over
-// that range: 1.8e-7 of the result's norm (2.9e-7 before).
+// B16 H32/8 S8192 D128 bf16 1399 -> 62 us (4.6 TB/s), float32 469 -> 64 us; B4 S3001 bf16 413 -> 15
+// us, float32 51 -> 16 us.  Measured error of float32 queries over that range: 1.8e-7 of the result's
+// norm (2.9e-7 before).
 
 #include "attn_common.h"
 #include "decode_merge.h"
