@@ -41,6 +41,7 @@
 #include "mfma_util.h"
 #include "lds_dma.h"
 #include "gt_rope_math.h"
+#include "prefill_order.h"
 
 #include <cmath>
 #include <type_traits>
@@ -131,13 +132,6 @@ __device__ inline void rope_rows(typename Mfma<T>::V8 *q, const float2 *tab, int
     }
 }
 
-// How a launch deals query tiles to workgroups.  kPairs: tiles p and nq-1-p of a head, one after
-// the other (equal work for every workgroup under the causal mask).  kSingle: one tile each, the
-// heaviest first (kHeadMajor: no causal mask, a head's tiles together); kFolded: one tile each where
-// all workgroups are resident at once, the heavier half first and then the lighter half from its
-// lightest, so that the two workgroups of a CU carry about the same together.
-enum TileOrder { kPairs = 0, kSingle = 1, kFolded = 2, kHeadMajor = 3 };
-
 // The tile(s) and head of workgroup x: qa (and then qb, when it differs).
 struct TileOf {
     int qa, qb;
@@ -162,23 +156,9 @@ __device__ inline TileOf tile_of(int order, int nq, int64_t BH, uint32_t x) {
     return {t, t, h0 + i % heads};
 }
 
-// Resident workgroups of the prefill kernels: two on each of the 256 CUs.
-constexpr int64_t kPrefillSlots = 512;
-
-// Pairs keep every workgroup's work equal and load Q and set up half as often, so they are taken
-// where their rounds over the slots are nearly full (causal fp16 B4 H32 L=S=2048 D128, two full
-// rounds: 162 us, single tiles 171).  Fewer workgroups than that leave slots empty, and a second
-// workgroup's MFMAs no longer cover the first one's softmax: single tiles then (same box, pairs
-// against single: bf16 B1 H32/8 L=S=2048 D128 68.2 -> 64.9 us, fp16 B1 H32/8 L=S=1024 32.2 -> 26.8,
-// fp16 B1 H8 L=S=3000 67.4 -> 58.8).  Without the causal mask all tiles weigh the same and single
-// ones always spread better (fp16 B4 H32/8 L500 S1500 D128 72.3 -> 60.3 us, with an (L,S) mask 132.8
-// -> 93.0; bf16 B2 H16 L300 S900 D64 34.5 -> 20.0; B4 H32 L=S=2048, many rounds: even).
 inline TileOrder tile_order(const AttnFwdArgs &a, int nq) {
-    const int64_t BH = a.B * a.H, pairs = (int64_t)((nq + 1) / 2) * BH;
-    if (!a.causal) return kHeadMajor;
-    const int64_t rounds = (pairs + kPrefillSlots - 1) / kPrefillSlots;
-    if (nq == 1 || pairs * 16 >= rounds * kPrefillSlots * 15) return kPairs;
-    return nq * BH <= kPrefillSlots ? kFolded : kSingle;
+    const bool light = a.out_dtype == GT_F16 && !a.o32 && !a.dropout;
+    return tile_order_of(a.causal != 0, light, (int)a.D, a.mt.cls || a.dropout, nq, a.B * a.H);
 }
 
 // Keys covered by query tile qt: the sequence's keys, or (causal) up to the tile's last row,

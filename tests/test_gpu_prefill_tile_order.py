@@ -16,12 +16,14 @@ from test_zz_no_alloc import noalloc
 pytestmark = pytest.mark.gpu
 
 
-def _order(causal, nq, heads):
+def _order(causal, light, D, nq, heads):
     """The rule under test, restated: 512 resident workgroups."""
     pairs = (nq + 1) // 2 * heads
+    slots = (pairs + 511) // 512 * 512
+    brief = nq in (4, 6, 8) and D in (64, 128)
     if not causal:
-        return "head major"
-    if nq == 1 or pairs * 16 >= (pairs + 511) // 512 * 512 * 15:
+        return "pairs" if brief and (light or D == 64) and pairs * 16 >= slots * 13 else "head major"
+    if nq == 1 or pairs * 16 >= slots * 15 or (brief and light and pairs >= 768):
         return "pairs"
     return "folded" if nq * heads <= 512 else "single"
 
@@ -36,9 +38,14 @@ def _order(causal, nq, heads):
     (torch.float16, 2, 5, 5, 128, 128, 128, True, "pairs"),
     (torch.bfloat16, 1, 6, 2, 400, 130, 128, False, "head major"),
     (torch.float16, 2, 8, 8, 385, 100, 64, False, "head major"),
+    (torch.float16, 6, 64, 8, 390, 70, 64, True, "pairs"),  # four tiles, one and a half rounds
+    (torch.bfloat16, 6, 64, 8, 390, 70, 64, True, "single"),
+    (torch.bfloat16, 4, 54, 54, 390, 70, 64, False, "pairs"),  # 13.5 of 16 slots
+    (torch.float16, 6, 35, 7, 500, 90, 128, False, "pairs"),
+    (torch.bfloat16, 6, 35, 7, 500, 90, 128, False, "head major"),
 ])
 def test_every_tile_order(dev, dtype, B, H, Hkv, L, S, D, causal, order):
-    assert _order(causal, (L + 127) // 128, B * H) == order
+    assert _order(causal, dtype == torch.float16, D, (L + 127) // 128, B * H) == order
     q, k, v = (randn((B, h, n, D), i + L, dtype) for i, (h, n) in enumerate(((H, L), (Hkv, S), (Hkv, S))))
     qd, kd, vd = (t.to(dev) for t in (q, k, v))
     got = torch.full((B, H, L, D), float("nan"), dtype=dtype, device=dev)
