@@ -368,7 +368,7 @@ def cpu_baseline():
 TRAFFIC_KERNELS = {
     "prefill": "prefill_fwd_kernelIDF16_Li128ELb1ELi0E",
     "decode": "decode_stream_kernelIDF16_Li128ELi4ELi0E",
-    "decode_q8_0": "decode_q8_lds_kernel<128, 4, 0>",
+    "decode_q8_0": "decode_q8_lds_kernelIDF16_Li128ELi4ELi0E",
 }
 TRAFFIC_FILE = ROOT / "profiles" / "hbm_traffic_prefill_decode.md"
 
@@ -497,10 +497,10 @@ TRACE_FILE = ROOT / "profiles" / "kernel_trace_bench_prefill_decode_q8_train_fp3
 TRACE_KERNELS = {
     "prefill": ["prefill_fwd_kernelIDF16_Li128ELb1ELi0E"],
     "decode": ["decode_stream_kernelIDF16_Li128ELi4ELi0E"],
-    "decode_q8_0": ["decode_q8_lds_kernel<128, 4, 0>"],
+    "decode_q8_0": ["decode_q8_lds_kernelIDF16_Li128ELi4ELi0E"],
     "train": ["prefill_fwd_kernelIDF16bLi64ELb1ELi4E", "bwd_dq_kernelIDF16bLi64ELb1ELi4E",
               "bwd_dkdv_kernelIDF16bLi64ELb1ELi4E"],
-    "fp32": ["generic_fwd"],
+    "fp32": ["prefill_f32_split_kernel<64, true, 0, false>"],
 }
 
 
