@@ -420,8 +420,8 @@ __global__ __launch_bounds__(64 * nw_of<D>(), DROP && (MASK == 1 || MASK == 2 ||
             // MTILE, tiles with other values: the mask's loads land during S = K.Q^T.  With two 32-key blocks
             // there are registers for them beside the scores; with four (head size 64) such tiles have a
             // product of their own, which keeps those registers out of the other tiles' way.  (After S, four
-            // loads at a time, they took a round trip per block: fp16 B4 H32 L=S=2048 D128 causal with
-            // float32 values 268 us, bf16 B8 H16 L=S=1024 D64 69.)
+            // loads at a time, they took a round trip per block: causal calls with float32 values, fp16 B4
+            // H32 L=S=2048 D128 268 us, now 242, bf16 B8 H16 L=S=1024 D64 69, now 60.)
             const float *mtrow = MTILE ? (const float *)a.mask + mtb * a.m_sb + (int64_t)min(lq, L - 1) * a.m_sl : nullptr;
             f32x4 mtv[MTILE && NKB == 2 ? NKB : 1][4];
             auto mt_load = [&](f32x4(*x)[4]) {  // (a copy's row pitch covers whole 4-key groups)

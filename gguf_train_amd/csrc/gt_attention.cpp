@@ -179,10 +179,11 @@ bool stage_mask(const gt_tensor *mask, int dev, int cd, AttnFwdArgs &a, Temps &t
 // than 0 and -inf are read in place).  Call with q, k, v and the options of `a` final.
 // What the tiles hold is not known here.  Where every one holds other values, half-precision masks lose
 // nothing (their pass replaces the conversion's: D64 B2 H16 L128 S512 fp16 35 -> 25 us, bf16 B8 H16
-// L=S=1024 causal 60.7 -> 61.9) and float32 ones the pass: nothing to see without the causal mask (D128 B4
-// H32/8 L500 S1500 fp16 119 -> 84), 5 to 12 us with it, when the mask as given took the same tile order
-// (D128 B4 H32 L=S=2048 fp16 230 -> 242, bf16 259 -> 261; B1 H32/8 L=S=4000 fp16 201 -> 220, bf16 232 ->
-// 233; D64 B8 H16 L=S=1024 fp16 52 -> 59, bf16 51 -> 60).  The same calls with a band or a finite blocked
+// L=S=1024 causal 60.7 -> 61.9) and float32 ones the pass, 3 to 12 us: nothing to see without the causal mask
+// unless the slots are full (D128 B4 H32/8 L500 S1500 fp16 119 -> 84; B16 H16 L=S=512 63 -> 65), but with it,
+// when the mask as given took the same tile order (D128 B4 H32 L=S=2048 fp16 230 -> 242, bf16 259 -> 261; B1
+// H32/8 L=S=4000 fp16 201 -> 220, bf16 232 -> 233; D64 B8 H16 L=S=1024 fp16 52 -> 59, bf16 51 -> 60; D128
+// with a mask per sequence 67 -> 78 and 74 -> 79).  The same calls with a band or a finite blocked
 // value gain more (fp16: 226 -> 174 and 180; 199 -> 160 and 161; 52 -> 37 and 41), and a window or
 // documents skip most tiles.
 // 1: staged, 0: not of this kind, -1: error.
